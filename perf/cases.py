@@ -65,6 +65,9 @@ def listed():
         # the adaptive tsunami remeshed before every step, between two outputs
         {"name": "adaptive_d16_26", "kind": "adaptive", "dmin": 16, "dmax": 26, "tol": 1.5e-3,
          "steps": 100, "toleranced": False},
+        # the same at an everyday size, on a coarse base mesh
+        {"name": "adaptive_d10_18", "kind": "adaptive", "dmin": 10, "dmax": 18, "tol": 8.0e-3,
+         "steps": 50, "toleranced": False},
         # one adjoint traversal of a depth-20 inversion
         {"name": "adjoint_step_d20", "kind": "adjoint", "scene": "tsunami", "depth": 20,
          "solver": "aug_riemann", "forward": True},

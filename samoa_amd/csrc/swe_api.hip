@@ -474,6 +474,7 @@ swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
     a.plotter = B.plotter;
     a.depth = B.depth;
     a.scen = B.d_scen;
+    a.scen0 = B.scen[0];  // read in place of the table when it is the only one
     a.chunk_scen = B.d_chunk_scen;
     a.slots = B.d_slots;
     a.part_min = B.d_part_min;

@@ -12,13 +12,17 @@
 //
 // Mapping.  A workgroup processes chunks of CH consecutive SFC cells of one
 // scenario (one thread per cell).  It stages the chunk's state in LDS, builds
-// a compact list of the edges it must solve (every edge to a higher-indexed
-// in-chunk partner once, edges to cells outside the chunk and domain-boundary
+// a compact list of the edges it must solve (each edge inside the chunk once,
+// from its left side; edges to cells outside the chunk and domain-boundary
 // edges by this chunk), solves them with one thread per list entry, scatters
 // both sides' fluxes into LDS, then updates its cells and reduces the CFL
 // candidate.  The Sierpinski order keeps almost every neighbour inside the
-// chunk, so ~1.5 Riemann solves per cell are done instead of 3, and halo
-// reads are L2 hits.  Chunks are dealt to XCDs in contiguous SFC ranges so
+// chunk, so ~1.6 Riemann solves per cell are done instead of 3, and halo
+// reads are L2 hits.  The edges that leave the chunk come last in the list: the
+// waves of inner edges neither wait for halo reads nor exchange the sides.
+// A wave whose edges are all clearly subcritical takes the short solver of
+// swe_riemann_clear.hpp (same results); the others are solved in a second
+// pass over the list.  Chunks are dealt to XCDs in contiguous SFC ranges so
 // each XCD's L2 holds the halos of its own chunks; a grid smaller than the
 // chunk count makes the launch persistent (grid-stride).
 //
@@ -38,6 +42,7 @@
 
 #include "swe_internal.hpp"
 #include "swe_riemann.hpp"
+#include "swe_riemann_clear.hpp"
 #include "swe_riemann_tol.hpp"
 
 namespace swe {
@@ -51,11 +56,47 @@ __device__ __forceinline__ double wave_min(double v) {
     return v;
 }
 
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// A pointer to memory that no kernel writes while this one runs, for scalar
+// loads from uniform addresses.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T *scalar(const T *p) {
+    return (const __attribute__((address_space(4))) T *)p;
+}
+
+// v_max_f64 without the quieting of signalling NaN that fmax adds.
+__device__ __forceinline__ double max_f64(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Lane 63 gets the maximum of values >= 0 over the wave (NaN only if every
+// value is one): row shifts by 1, 2, 4 and 8, then the rows' last lanes
+// broadcast to the next row and half; a lane without a source reads 0.
+__device__ __forceinline__ double wave_max(double v) {
+    auto step = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        v = max_f64(v, __hiloint2double(
+                           __builtin_amdgcn_update_dpp(0, __double2hiint(v), C, 0xf, 0xf, true),
+                           __builtin_amdgcn_update_dpp(0, __double2loint(v), C, 0xf, 0xf, true)));
+    };
+    step(std::integral_constant<int, 0x111>{});
+    step(std::integral_constant<int, 0x112>{});
+    step(std::integral_constant<int, 0x114>{});
+    step(std::integral_constant<int, 0x118>{});
+    step(std::integral_constant<int, 0x142>{});
+    step(std::integral_constant<int, 0x143>{});
     return v;
 }
+
+// Lanes of the mask below this one.
+__device__ __forceinline__ int lanes_below(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// Flags of the edge list's entries.
+constexpr uint32_t LEAVES = 1u << 31, BOUNDARY = 1u << 30;
 
 // Four waves per SIMD (at most 128 VGPRs, a few spilled) outrun three
 // unspilled ones: the LDS of four 256-cell workgroups fits a CU.
@@ -69,71 +110,73 @@ __device__ __forceinline__ int wave_sum_i(int v) {
 // registers.
 template <int SOLVER, int CH, bool JUMPS, bool RAW = false, bool TOL = false>
 __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void euler_step_kernel(
-    StepArgs a) {
+    StepArgs args) {
     static_assert(!(RAW && TOL), "the toleranced kernel reads packed neighbours");
-    static_assert(!TOL || SOLVER == 0 || SOLVER == 1, "toleranced GeoClaw solvers only");
+    constexpr bool GEOCLAW = SOLVER == 0 || SOLVER == 1;
+    static_assert(!TOL || GEOCLAW, "toleranced GeoClaw solvers only");
+    constexpr bool CLEAR = GEOCLAW && !TOL;  // clear_flux where a wave's edges allow it
     constexpr int NW = CH / 64;
-    __shared__ double s_q[4][CH];        // eta, hu, hv, b of the chunk (TOL: h, wu, wv, b)
-    __shared__ double s_x[TOL ? CH : 1];  // TOL: sqrt(g h) (0 when dry)
-    __shared__ double s_f[4][3][CH];     // flux (h, hu, hv, s) per (edge, cell)
-    __shared__ int32_t s_nbr[3][CH];     // packed neighbour (o << 2 | back edge)
-    __shared__ int8_t s_plot[CH];
-    __shared__ uint16_t s_list[3 * CH];  // (local cell << 2) | edge
-    // JUMPS: elevation-jump bits per (edge, cell), from the edge loop, which
-    // holds both states
-    __shared__ uint8_t s_jb[JUMPS ? 3 : 1][JUMPS ? CH : 1];
+    __shared__ double s_q[4][CH];  // eta, hu, hv, b of the chunk (TOL: h, wu, wv, b)
+    // CLEAR: 1/h and sqrt(g h) of each cell (clear_cell); TOL: sqrt(g h) (0 when dry)
+    __shared__ double s_x[CLEAR ? 2 : 1][CLEAR || TOL ? CH : 1];
+    __shared__ double s_f[4][3][CH];  // flux (h, hu, hv, s) per (edge, cell)
+    // The edges to solve: those inside the chunk first, then those leaving it
+    // (to other chunks or the boundary), then the packed neighbours of the
+    // latter.  A chunk of m cells of a validated mesh has at least m - 1
+    // inner edges (consecutive cells share one), so at most m + 2 leave it:
+    // inner + 2 leaving = (3 m + 3 leaving) / 2 <= 3 m + 3 entries.  RAW
+    // meshes are not validated; their neighbours are read again instead.
+    __shared__ uint32_t s_list[3 * CH + 4];
+    __shared__ uint32_t s_jb[JUMPS ? CH / 16 : 1];  // elevation-jump bits, 2 per cell
     __shared__ int s_wsum[NW];
-    __shared__ double s_wmin[NW];
+    __shared__ double s_wmax[NW];
     __shared__ int s_wref[NW];
     // geometry tables in LDS: the per-lane indexed reads would otherwise be
-    // global loads that every edge waits for (the toleranced kernel reads
-    // them from constant memory: its LDS holds four workgroups per CU only
-    // without them)
-    __shared__ double s_normal[TOL ? 1 : 17 * 3 * 2];
-    __shared__ double s_leg[TOL ? 1 : 64];
-    auto normal_at = [&](int i) -> double {
-        if constexpr (TOL) return c_normal[i];
-        else return s_normal[i];
-    };
-    auto leg_at = [&](int i) -> double {
-        if constexpr (TOL) return c_leg[i];
-        else return s_leg[i];
-    };
+    // global loads that every edge waits for
+    __shared__ double s_dir[8][2];  // the unit vectors at multiples of 45 degrees
+    __shared__ double s_leg[64];
 
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
-    const double g = a.g, inv16g = a.inv16g;
-    if constexpr (!TOL) {
-        for (int i = t; i < 17 * 3 * 2; i += CH) s_normal[i] = c_normal[i];
-        for (int i = t; i < 64; i += CH) s_leg[i] = c_leg[i];
-        __syncthreads();
-    }
+    // the hypotenuse normals of plotter types 1..8 point to 90, 135, ... degrees
+    if (t < 16) s_dir[t >> 1][t & 1] = c_normal[((((t >> 1) - 2) & 7) + 9) * 6 + 2 + (t & 1)];
+    for (int i = t; i < 64; i += CH) s_leg[i] = c_leg[i];
 
     // XCD-aware order: virtual block v runs on XCD v % 8 (the dispatcher deals
     // workgroups round robin and the grid is a multiple of 8); XCD x owns a
     // contiguous range of chunks.
-    const int64_t nchunks = a.nchunks;
-    const int64_t q = nchunks / 8, r = nchunks % 8;
-    const int64_t nvirt = 8 * ((nchunks + 7) / 8);
-    for (int64_t v = blockIdx.x; v < nvirt; v += gridDim.x) {
-        const int64_t xcd = v % 8, i = v / 8;
+    // (there are fewer than 2^31 chunks)
+    const uint32_t nchunks = (uint32_t)args.nchunks, q = nchunks / 8, r = nchunks % 8;
+    const uint32_t nvirt = 8 * ((nchunks + 7) / 8);
+    for (uint32_t v = blockIdx.x; v < nvirt; v += gridDim.x) {
+        const uint32_t xcd = v % 8, i = v / 8;
         if (i >= q + (xcd < r ? 1 : 0)) continue;  // uniform across the workgroup
-        const int64_t chunk = xcd * q + (xcd < r ? xcd : r) + i;
+        const uint32_t chunk = xcd * q + (xcd < r ? xcd : r) + i;
+        // The arguments are read where they are used, for each chunk (the
+        // empty asm hides that the address is the same every time): held
+        // across the loop, they and what is derived from them outgrow the
+        // scalar registers, and every wave moved them to vector lanes first.
+        auto ap = (const __attribute__((address_space(4))) StepArgs *)
+            __builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(ap));
+        const auto &a = *ap;
+        const double g = a.g, inv16g = a.inv16g;
         // Raised wave priority from here to the edge loop: the chunk's
         // descriptor and staging loads, and the edge list, are a chain of
         // memory round trips and barriers; issued ahead of the other waves'
         // solver arithmetic, they overlap it (3-5 % off the step).
         __builtin_amdgcn_s_setprio(2);
-        const int s = a.chunk_scen ? a.chunk_scen[chunk] : 0;
-        const Scen sc = RAW ? a.scen0 : a.scen[s];
+        // What is uniform is read through the scalar cache; one scenario's
+        // table entry comes with the arguments, so that its state loads do
+        // not wait for a table read.
+        const int s = !RAW && a.chunk_scen ? scalar(a.chunk_scen)[chunk] : 0;
+        const auto *const sp = !RAW && a.chunk_scen ? scalar(a.scen) + s : &a.scen0;
+        const auto &sc = *sp;
         // The state and topology arrays are addressed from per-scenario
         // (gs_*) and per-chunk (c_*) base pointers that are uniform across
-        // the workgroup.  Cell indices are 64-bit in the exact kernel and
-        // 32-bit in the toleranced one (a scenario holds at most 2^29 cells):
-        // measured, each is the faster of the two for that kernel (by 3-4 %
-        // and by about 1 %).
-        using Index = std::conditional_t<TOL, int32_t, int64_t>;
-        const Index lbase = (Index)((chunk - sc.chunk_off) * CH);  // first cell of the chunk
+        // the workgroup; cell indices are 32-bit (a scenario holds at most
+        // 2^29 cells).
+        const int32_t lbase = (int32_t)(chunk - (uint32_t)sc.chunk_off) * CH;  // first cell of the chunk
         const int cnt = (int)((sc.n - lbase) < CH ? (sc.n - lbase) : CH);
         const bool active = t < cnt;
         const int64_t gs = sc.cell_off, gt = sc.topo_off;  // state / topology offsets
@@ -145,39 +188,40 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         const int8_t *const c_plot = a.plotter + gt + lbase;
         const int8_t *const c_depth = a.depth + gt + lbase;
         const int64_t c_out = gs + lbase;  // first output cell of the chunk
-        const double dt = a.device_dt ? a.slots[s].dt : (a.dt_host ? a.dt_host[s] : a.dt);
+        const double dt = a.device_dt ? scalar(a.slots)[s].dt
+                                      : (a.dt_host ? scalar(a.dt_host)[s] : a.dt);
         const double drytol = sc.drytol;
 
         int32_t nb[3] = {-1, -1, -1};
-        int8_t plot = 1;
+        int plot = 1;
         double my_e = 0.0, my_u = 0.0, my_v = 0.0;  // TOL: this thread's cell state
         if (active) {
+            // every load goes out before the arithmetic that waits for the state
+            const double e = c_eta[t], u = c_hu[t], vv = c_hv[t], bb = c_b[t];
+            nb[0] = c_nbr[3 * t];
+            nb[1] = c_nbr[3 * t + 1];
+            nb[2] = c_nbr[3 * t + 2];
+            plot = c_plot[t];
             if constexpr (TOL) {
-                // the topology loads go out with the state's, before the
-                // arithmetic that waits for the state
-                my_e = c_eta[t];
-                my_u = c_hu[t];
-                my_v = c_hv[t];
-                const double my_b = c_b[t];
-                nb[0] = c_nbr[3 * t];
-                nb[1] = c_nbr[3 * t + 1];
-                nb[2] = c_nbr[3 * t + 2];
-                plot = c_plot[t];
-                const tol::CellQ cq = tol::cell_q(my_e, my_u, my_v, my_b, drytol, g);
+                my_e = e;
+                my_u = u;
+                my_v = vv;
+                const tol::CellQ cq = tol::cell_q(e, u, vv, bb, drytol, g);
                 s_q[0][t] = cq.h;
                 s_q[1][t] = cq.wu;
                 s_q[2][t] = cq.wv;
                 s_q[3][t] = cq.b;
-                s_x[t] = cq.sq;
+                s_x[0][t] = cq.sq;
             } else {
-                s_q[0][t] = c_eta[t];
-                s_q[1][t] = c_hu[t];
-                s_q[2][t] = c_hv[t];
-                s_q[3][t] = c_b[t];
-                nb[0] = c_nbr[3 * t];
-                nb[1] = c_nbr[3 * t + 1];
-                nb[2] = c_nbr[3 * t + 2];
-                plot = c_plot[t];
+                s_q[0][t] = e;
+                s_q[1][t] = u;
+                s_q[2][t] = vv;
+                s_q[3][t] = bb;
+                if constexpr (CLEAR) {
+                    const ClearCell k = clear_cell(e, u, vv, bb, drytol, g);
+                    s_x[0][t] = k.r;
+                    s_x[1][t] = k.c;
+                }
             }
             if (RAW) {  // a neighbour outside the mesh reads as the boundary
 #pragma unroll
@@ -185,209 +229,211 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                     if ((uint32_t)nb[k] >= (uint64_t)sc.n) nb[k] = -1;
             }
         }
-        s_nbr[0][t] = nb[0];
-        s_nbr[1][t] = nb[1];
-        s_nbr[2][t] = nb[2];
-        s_plot[t] = plot;
+        // RAW: the chunk's neighbours, for the back edges; the flux slots are
+        // not written before the edge loop
+        int32_t *const s_nbr = reinterpret_cast<int32_t *>(&s_f[0][0][0]);
+        if (RAW) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s_nbr[k * CH + t] = nb[k];
+        }
+        if (JUMPS && t < CH / 16) s_jb[t] = 0;
 
-        // Edges this thread's cell must solve: boundary, halo, or in-chunk
-        // with a higher-indexed partner.
-        int own = 0;
+        // Edges this thread's cell must solve: those leaving the chunk, and
+        // the inner ones whose other cell the traversal visits later.  Inner
+        // edges are so solved from their left side.
+        int inner = 0, leave = 0;
         if (active) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const int32_t p = nb[k];
-                if constexpr (TOL) {
-                    const int lo = (p >> 2) - lbase;  // chunk-local neighbour
-                    const bool inside = p >= 0 && (uint32_t)lo < (uint32_t)cnt;
-                    if (!inside || lo > t) own |= 1 << k;
-                } else {
-                    const int64_t o = (int64_t)(RAW ? p : p >> 2);
-                    const bool inside = p >= 0 && o >= lbase && o < lbase + cnt;
-                    if (!inside || o > lbase + t) own |= 1 << k;
-                }
+                const int lo = (RAW ? p : p >> 2) - lbase;  // chunk-local neighbour
+                const bool inside = p >= 0 && (uint32_t)lo < (uint32_t)cnt;
+                if (!inside) leave |= 1 << k;
+                else if (a.forward ? lo > t : lo < t) inner |= 1 << k;
             }
         }
-        const int nown = __popc(own);
-        // workgroup exclusive prefix of nown via ballots (nown in 0..3)
-        const uint64_t b0 = __ballot(nown & 1), b1 = __ballot(nown & 2);
-        const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-        const int wpre = __popcll(b0 & lt) + 2 * __popcll(b1 & lt);
-        if (lane == 0) s_wsum[wave] = __popcll(b0) + 2 * __popcll(b1);
+        // workgroup exclusive prefixes of both counts (0..3 each) via ballots,
+        // packed: inner in the low half, leaving in the high half
+        const int nin = __popc(inner), nout = __popc(leave);
+        const uint64_t i0 = __ballot(nin & 1), i1 = __ballot(nin & 2);
+        const uint64_t o0 = __ballot(nout & 1), o1 = __ballot(nout & 2);
+        const int wpre = lanes_below(i0) + 2 * lanes_below(i1) +
+                         ((lanes_below(o0) + 2 * lanes_below(o1)) << 16);
+        if (lane == 0)
+            s_wsum[wave] = __popcll(i0) + 2 * __popcll(i1) +
+                           ((__popcll(o0) + 2 * __popcll(o1)) << 16);
         __syncthreads();
-        int pre = wpre, total = 0;
+        int pre = wpre, sum = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             const int ws = s_wsum[w];
             pre += w < wave ? ws : 0;
-            total += ws;
+            sum += ws;
         }
+        const int n_inner = sum & 0xffff, total = n_inner + (sum >> 16);
+        int pi = pre & 0xffff, po = n_inner + (pre >> 16);
+        // outward normal of edge k: plotter type p > 0 turns the normals at
+        // 180 + 45 p, 45 + 45 p and 270 + 45 p degrees, p < 0 mirrors the legs
+        const int turn = plot < 0 ? -plot : plot;
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (own & (1 << k)) s_list[pre++] = (uint16_t)((t << 2) | k);
+        for (int k = 0; k < 3; ++k) {
+            const int d0 = k == 1 ? 1 : ((k == 0) == (plot > 0) ? 4 : 6);
+            const int32_t p = nb[k];
+            const bool in = inner & (1 << k), out = leave & (1 << k);
+            const int lo = (RAW ? p : p >> 2) - lbase;
+            int ko = p & 3;
+            // a plain neighbour's edge back to this cell (two cells of a
+            // conforming mesh share at most one edge)
+            if (RAW && in) ko = s_nbr[lo] == lbase + t ? 0 : (s_nbr[CH + lo] == lbase + t ? 1 : 2);
+            const uint32_t other = in ? ((uint32_t)lo << 11) | ((uint32_t)ko << 20)
+                                      : LEAVES | (p < 0 ? BOUNDARY : 0u);
+            if (in || out)
+                s_list[in ? pi : po] = (uint32_t)t | ((uint32_t)k << 9) |
+                                       ((uint32_t)((turn + d0) & 7) << 22) | other;
+            if (!RAW && out) s_list[po + total - n_inner] = (uint32_t)p;
+            pi += in ? 1 : 0;
+            po += out ? 1 : 0;
+        }
         __syncthreads();
 
         __builtin_amdgcn_s_setprio(0);
-        for (int e = t; e < total; e += CH) {
-            if constexpr (TOL) {
-                const int ent = s_list[e];
-                const int lc = ent >> 2, k = ent & 3;
-                const int32_t p = s_nbr[k][lc];
-                const int pi = s_plot[lc] + 8;
-                const double nx = normal_at((pi * 3 + k) * 2), ny = normal_at((pi * 3 + k) * 2 + 1);
-                const double hC = s_q[0][lc], uC = s_q[1][lc], vC = s_q[2][lc], bC = s_q[3][lc];
-                const double sqC = s_x[lc];
-                const bool bnd = p < 0;
-                const int32_t o = RAW ? p : p >> 2;  // the neighbour (not read when bnd)
-                const int lo = o - lbase;
-                const bool inside = !bnd && (uint32_t)lo < (uint32_t)cnt;
-                double hO, uO, vO, bO, sqO;
-                if (bnd) {  // ghost: the cell itself, velocity mirrored at a wall
-                    hO = hC;
-                    bO = bC;
-                    sqO = sqC;
-                    uO = uC;
-                    vO = vC;
-                    if (a.bc == 1) {
-                        const double dp = uC * nx + vC * ny;
-                        uO = uC - (2.0 * dp) * nx;
-                        vO = vC - (2.0 * dp) * ny;
-                    }
-                } else if (inside) {
-                    hO = s_q[0][lo];
-                    uO = s_q[1][lo];
-                    vO = s_q[2][lo];
-                    bO = s_q[3][lo];
-                    sqO = s_x[lo];
-                } else {
-                    const tol::CellQ cq =
-                        tol::cell_q(gs_eta[o], gs_hu[o], gs_hv[o], gs_b[o], drytol, g);
-                    hO = cq.h;
-                    uO = cq.wu;
-                    vO = cq.wv;
-                    bO = cq.b;
-                    sqO = cq.sq;
-                }
-                // the left state as in the exact path: the operands of the
-                // well-balancing sums (b + h of the right cell first) round
-                // with the side they are on, and in deep water those
-                // roundings are the largest part of a momentum update
-                const bool c_left = bnd || (a.forward ? (lc < lo) : (lc > lo));
-                const double sx = c_left ? nx : -nx, sy = c_left ? ny : -ny;
-                Flux fL, fR;
-                tol::edge_flux<SOLVER>(sx, sy, c_left ? hC : hO, c_left ? uC : uO,
-                                       c_left ? vC : vO, c_left ? bC : bO, c_left ? sqC : sqO,
-                                       c_left ? hO : hC, c_left ? uO : uC, c_left ? vO : vC,
-                                       c_left ? bO : bC, c_left ? sqO : sqC, drytol, g, inv16g,
-                                       fL, fR);
-                const Flux fc = c_left ? fL : fR;
-                const Flux fo = c_left ? fR : fL;
-                s_f[0][k][lc] = fc.h;
-                s_f[1][k][lc] = fc.hu;
-                s_f[2][k][lc] = fc.hv;
-                s_f[3][k][lc] = fc.s;
-                uint8_t jb = 0;
-                if constexpr (JUMPS) {
-                    // as in the exact path below, with eta = h + b
-                    if (!bnd && hC > drytol && hO > drytol) {
-                        const double jd = fabs((hC + bC) - (hO + bO));
-                        jb = (uint8_t)((jd > a.jump_refine ? 1 : 0) |
-                                       (jd >= a.jump_coarsen ? 2 : 0));
-                    }
-                    s_jb[k][lc] = jb;
-                }
-                if (inside) {
-                    const int ko = p & 3;
-                    s_f[0][ko][lo] = fo.h;
-                    s_f[1][ko][lo] = fo.hu;
-                    s_f[2][ko][lo] = fo.hv;
-                    s_f[3][ko][lo] = fo.s;
-                    if constexpr (JUMPS) s_jb[ko][lo] = jb;
-                }
-                continue;
-            }
-            const int ent = s_list[e];
-            const int lc = ent >> 2, k = ent & 3;
-            const int64_t cc = lbase + lc;
-            const int32_t p = s_nbr[k][lc];
-            const int pi = s_plot[lc] + 8;
-            const double nx = normal_at((pi * 3 + k) * 2), ny = normal_at((pi * 3 + k) * 2 + 1);
-            const double qe = s_q[0][lc], qu = s_q[1][lc], qv = s_q[2][lc], qb = s_q[3][lc];
-            const bool bnd = p < 0;
-            const int64_t o = bnd ? cc : (int64_t)(RAW ? p : p >> 2);
-            const bool inside = !bnd && o >= lbase && o < lbase + cnt;
-            const int lo = (int)(o - lbase);  // chunk-local neighbour (used when inside)
-            // the neighbour's edge back to this cell: packed with it, or for
-            // plain neighbours found among the in-chunk neighbour's own
-            // (two cells of a conforming mesh share at most one edge)
-            int ko = p & 3;
-            if (RAW && inside) ko = s_nbr[0][lo] == (int32_t)cc ? 0 : (s_nbr[1][lo] == (int32_t)cc ? 1 : 2);
-            double oe, ou, ov, ob;
-            if (bnd) {  // ghost state of bnd_skeleton_scalar_op (outflow copy or mirror)
-                oe = qe;
-                ob = qb;
-                ou = qu;
-                ov = qv;
+        // One pass over the list.  FIRST: a CLEAR kernel's pass with clear_flux,
+        // which leaves the rounds (of CH entries) where one of a wave's edges
+        // is not clear to a second pass with the general solver; returns their
+        // bits, the same for the whole wave.  A pass of its own keeps the
+        // general solver's registers from adding to the shortcut's.
+        auto solve = [&](auto first_pass, uint32_t rounds) -> uint32_t {
+        constexpr bool FIRST = decltype(first_pass)::value;
+        constexpr bool SHORT = CLEAR && FIRST;
+        uint32_t rest = 0, bit = 1;
+        for (int e = t; e < total; e += CH, bit <<= 1) {
+            if (!FIRST && !(rounds & bit)) continue;
+            const uint32_t ent = s_list[e];
+            const int lc = ent & 511, k = (ent >> 9) & 3, dir = (ent >> 22) & 7;
+            double nx = s_dir[dir][0], ny = s_dir[dir][1];
+            // the two cells' quantities: left and right for an inner edge;
+            // one that leaves the chunk may need them exchanged
+            double L[6] = {}, R[6] = {};
+#pragma unroll
+            for (int m = 0; m < 4; ++m) L[m] = s_q[m][lc];
+            if (SHORT || TOL) L[4] = s_x[0][lc];
+            if (SHORT) L[5] = s_x[CLEAR ? 1 : 0][lc];
+            const bool inside = !(ent & LEAVES);
+            const int lo = (ent >> 11) & 511;
+            bool flip = false;
+            uint32_t jb = 0;
+            if (inside) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) R[m] = s_q[m][lo];
+                if (SHORT || TOL) R[4] = s_x[0][lo];
+                if (SHORT) R[5] = s_x[CLEAR ? 1 : 0][lo];
+            } else if (ent & BOUNDARY) {
+                // ghost state of bnd_skeleton_scalar_op (outflow copy or mirror)
+#pragma unroll
+                for (int m = 0; m < 6; ++m) R[m] = L[m];
                 if (a.bc == 1) {
-                    const double dp = qu * nx + qv * ny;
-                    ou = qu - (2.0 * dp) * nx;
-                    ov = qv - (2.0 * dp) * ny;
+                    const double dp = L[1] * nx + L[2] * ny;
+                    R[1] = L[1] - (2.0 * dp) * nx;
+                    R[2] = L[2] - (2.0 * dp) * ny;
                 }
-            } else if (inside) {
-                oe = s_q[0][lo];
-                ou = s_q[1][lo];
-                ov = s_q[2][lo];
-                ob = s_q[3][lo];
             } else {
-                oe = gs_eta[o];
-                ou = gs_hu[o];
-                ov = gs_hv[o];
-                ob = gs_b[o];
+                const int32_t p = RAW ? c_nbr[3 * lc + k] : (int32_t)s_list[e + total - n_inner];
+                const int32_t o = RAW ? p : p >> 2;
+                R[0] = gs_eta[o];
+                R[1] = gs_hu[o];
+                R[2] = gs_hv[o];
+                R[3] = gs_b[o];
+                if constexpr (TOL) {
+                    const tol::CellQ cq = tol::cell_q(R[0], R[1], R[2], R[3], drytol, g);
+                    R[0] = cq.h;
+                    R[1] = cq.wu;
+                    R[2] = cq.wv;
+                    R[4] = cq.sq;
+                }
+                if constexpr (SHORT) {
+                    const ClearCell x = clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+                    R[4] = x.r;
+                    R[5] = x.c;
+                }
+                flip = a.forward ? o < lbase : o > lbase;  // the other cell comes first
             }
-            // one solver call per entry: the left state is this cell on the
-            // boundary and when it comes first in the traversal direction
-            const bool c_left = bnd || (a.forward ? (cc < o) : (cc > o));
-            const double sx = c_left ? nx : -nx, sy = c_left ? ny : -ny;
-            Flux fL, fR;
-            edge_flux<SOLVER>(sx, sy, c_left ? qe : oe, c_left ? qu : ou, c_left ? qv : ov,
-                              c_left ? qb : ob, c_left ? oe : qe, c_left ? ou : qu,
-                              c_left ? ov : qv, c_left ? ob : qb, drytol, g, inv16g, fL, fR);
-            const Flux fc = c_left ? fL : fR;
-            s_f[0][k][lc] = fc.h;
-            s_f[1][k][lc] = fc.hu;
-            s_f[2][k][lc] = fc.hv;
-            s_f[3][k][lc] = fc.s;
-            uint8_t jb = 0;
-            if constexpr (JUMPS) {
+            if constexpr (JUMPS && FIRST) {
                 // the elevation jump across an edge between two wet cells:
                 // bit 0 if above the refinement tolerance, bit 1 if not below
                 // the coarsening tolerance (a NaN jump sets neither); the
                 // same for both cells, as |a - b| = |b - a|
-                if (!bnd && qe - qb > drytol && oe - ob > drytol) {
-                    const double jd = fabs(qe - oe);
-                    jb = (uint8_t)((jd > a.jump_refine ? 1 : 0) | (jd >= a.jump_coarsen ? 2 : 0));
+                const double hl = TOL ? L[0] : L[0] - L[3], hr = TOL ? R[0] : R[0] - R[3];
+                const double jd = TOL ? fabs((L[0] + L[3]) - (R[0] + R[3])) : fabs(L[0] - R[0]);
+                if (!(ent & BOUNDARY) && hl > drytol && hr > drytol)
+                    jb = (jd > a.jump_refine ? 1u : 0u) | (jd >= a.jump_coarsen ? 2u : 0u);
+                if (jb) {
+                    atomicOr(&s_jb[lc >> 4], jb << (2 * (lc & 15)));
+                    if (inside) atomicOr(&s_jb[lo >> 4], jb << (2 * (lo & 15)));
                 }
-                s_jb[k][lc] = jb;
             }
+            const bool flips = __ballot(flip) != 0;  // no wave of inner edges does
+            if (flips) {
+#pragma unroll
+                for (int m = 0; m < 6; ++m) {
+                    const double x = L[m];
+                    L[m] = flip ? R[m] : x;
+                    R[m] = flip ? x : R[m];
+                }
+                nx = flip ? -nx : nx;
+                ny = flip ? -ny : ny;
+            }
+            Flux fL, fR;
+            if constexpr (TOL) {
+                tol::edge_flux<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], L[4], R[0], R[1], R[2], R[3],
+                                       R[4], drytol, g, inv16g, fL, fR);
+            } else if constexpr (SHORT) {
+                const double hL = L[0] - L[3], hR = R[0] - R[3];
+                const ClearEdge ce = clear_edge(nx, ny, hL, L[1], L[2], L[4], hR, R[1], R[2], R[4]);
+                const bool dead = hL <= drytol && hR <= drytol;
+                if (__ballot(!dead && !is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5])) != 0) {
+                    rest |= bit;
+                    continue;
+                }
+                clear_flux<SOLVER>(nx, ny, ce, hL, L[3], L[5], hR, R[3], R[5], g, fL, fR);
+                if (__ballot(dead) != 0 && dead) fL = fR = Flux{0.0, 0.0, 0.0, 0.0};
+            } else {
+                edge_flux<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], R[0], R[1], R[2], R[3], drytol, g,
+                                  inv16g, fL, fR);
+            }
+            if (flips && flip) fL = fR;
+            s_f[0][k][lc] = fL.h;
+            s_f[1][k][lc] = fL.hu;
+            s_f[2][k][lc] = fL.hv;
+            s_f[3][k][lc] = fL.s;
             if (inside) {
-                const Flux fo = c_left ? fR : fL;
-                s_f[0][ko][lo] = fo.h;
-                s_f[1][ko][lo] = fo.hu;
-                s_f[2][ko][lo] = fo.hv;
-                s_f[3][ko][lo] = fo.s;
-                if constexpr (JUMPS) s_jb[ko][lo] = jb;
+                const int ko = (ent >> 20) & 3;
+                s_f[0][ko][lo] = fR.h;
+                s_f[1][ko][lo] = fR.hu;
+                s_f[2][ko][lo] = fR.hv;
+                s_f[3][ko][lo] = fR.s;
             }
+        }
+        return rest;
+        };
+        const uint32_t rest = solve(std::true_type{}, 0u);
+        if constexpr (CLEAR) {
+            if (rest) (void)solve(std::false_type{}, rest);
         }
         __syncthreads();
 
         // cell update: volume_op + cell_update_op
-        double cand = 1.7976931348623157e308;  // huge(1.0_SR), pre_traversal_op :139
-        int refined = 0;
+        // The CFL candidate of a cell is fl(volume / sv), volume = S^2 2^-(d+1):
+        // scaling by a power of two is exact and the rounded quotient falls
+        // as the divisor grows, so the chunk's minimum is the quotient of S^2
+        // and the largest sv 2^(d+1) (without cells: huge(1.0_SR),
+        // pre_traversal_op :139)
+        double speed = 0.0;
+        bool refined = false;
         if (active) {
             const int d = sc.depth >= 0 ? sc.depth : (int)c_depth[t];
             const double S = sc.scaling;
             const double volume = (S * S) * ldexp(1.0, -(d + 1));
-            const double lleg = S * leg_at(d + 1), lhyp = S * leg_at(d);
+            const double lleg = S * s_leg[d + 1], lhyp = S * s_leg[d];
             const int k0 = a.forward ? 0 : 2, k2 = a.forward ? 2 : 0;
             double dh = 0.0, d1 = 0.0, d2 = 0.0, sv = 0.0;
             dh = dh + lleg * s_f[0][k0][t];
@@ -411,10 +457,10 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 // not below the coarsening tolerance.  j = the largest jump
                 // (0 without a wet neighbour): j > tol if some edge's is,
                 // j < tol if every edge's is and tol > 0.
-                const int jb = s_jb[0][t] | s_jb[1][t] | s_jb[2][t];
+                const int jb = (s_jb[t >> 4] >> (2 * (t & 15))) & 3;
                 if (d < sc.dmax && (jb & 1)) {
                     rf = 1;
-                    refined = 1;
+                    refined = true;
                 } else if (d > sc.dmin && !(jb & 2) && a.jump_coarsen > 0.0) {
                     rf = -1;
                 }
@@ -422,13 +468,13 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 const double dq = fabs(dh);
                 if (d < sc.dmax && dq > sc.refine_thr) {
                     rf = 1;
-                    refined = 1;
+                    refined = true;
                 } else if (d > sc.dmin && dq < sc.refine_thr / 8.0) {
                     rf = -1;
                 }
             }
             if (a.refine) a.refine[c_out + t] = rf;
-            cand = volume / sv;
+            speed = ldexp(sv, d + 1);
             const double scale = -dt / volume;
             dh = scale * dh;
             d1 = scale * d1;
@@ -461,22 +507,22 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
 
         // CFL minimum and refinement count of the chunk (post_traversal_grid_op
         // :117-118); the finalize kernel reduces the chunks of each scenario.
-        const double wmin = wave_min(cand);
-        const int wref = wave_sum_i(refined);
-        if (lane == 0) {
-            s_wmin[wave] = wmin;
+        const double wmax = wave_max(speed);
+        const int wref = __popcll(__ballot(refined));
+        if (lane == 63) {
+            s_wmax[wave] = wmax;
             s_wref[wave] = wref;
         }
         __syncthreads();
         if (t == 0) {
-            double m = s_wmin[0];
+            double m = s_wmax[0];
             int rsum = s_wref[0];
 #pragma unroll
             for (int w = 1; w < NW; ++w) {
-                m = dmin2(m, s_wmin[w]);
+                m = max_f64(m, s_wmax[w]);
                 rsum += s_wref[w];
             }
-            a.part_min[chunk] = m;
+            a.part_min[chunk] = (sc.scaling * sc.scaling) / m;
             a.part_nref[chunk] = rsum;
         }
         __syncthreads();  // LDS is reused by the next chunk

@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 
 #include "swe_riemann.hpp"
+#include "swe_riemann_clear.hpp"
 
 namespace swe {
 namespace tol {
@@ -339,6 +340,86 @@ __device__ __forceinline__ void edge_flux(double nx, double ny, double hL, doubl
     fR.h = netR[0];
     fR.hu = netR[1] * nx - netR[2] * ny;
     fR.hv = netR[1] * ny + netR[2] * nx;
+    fR.s = s;
+}
+
+// An edge whose general solve takes no branch that matters, as in
+// swe_riemann_clear.hpp (both sides wet: the roots are above 0.06; their bound
+// keeps the test's rounding below its margin, and a NaN or an infinity fails).
+template <int SOLVER>
+__device__ __forceinline__ bool is_clear(double uL, double uR, double sqL, double sqR) {
+    return swe::is_clear<SOLVER>(uL, uR, sqL, sqR) && sqL + sqR < 0x1p26;
+}
+
+// edge_flux<SOLVER> on a clear edge: the same operations without riemanntype,
+// the bounds on deldelh (except near them) and the wave split's tests; the
+// two divisions by s1s2bar share a reciprocal.  u, v: normal and tangential
+// velocities.  The d21 tsunami step (4.2 M cells): 148 us with the general
+// solver for every edge, 124 us with this one.
+template <int SOLVER>
+__device__ __forceinline__ void clear_flux(double nx, double ny, double hL, double uL, double vL,
+                                           double bL, double sqL, double hR, double uR, double vR,
+                                           double bR, double sqR, double g, Flux &fL, Flux &fR) {
+    const double huL = hL * uL, huR = hR * uR;
+    const double hsum = hR + hL, usum = uL + uR, uu = uL * uR;
+    const double delh = hR - hL, delhu = huR - huL, delb = bR - bL;
+    const double delphi = ((delhu * usum - uu * delh) + ((0.5 * g) * (((bR + hR) - bL) - hL)) * hsum) -
+                          ((0.5 * g) * hsum) * delb;
+    const double uhat = (sqL * uL + sqR * uR) * rcp(sqR + sqL);
+    const double chat = sqrt0((g * 0.5) * hsum);
+    const double l0 = fmin(uL - sqL, uhat - chat);
+    const double l2 = fmax(uR + sqR, uhat + chat);
+    const double rspan = rcp(l2 - l0);
+    double l1 = 0.5 * (l0 + l2);
+    double f00, f10, f11, f12, f02;
+    if (SOLVER == 1) {  // riemann_fwave, riemannsolvers.f:446-500
+        const double dec = delphi - -(((g * 0.5) * hsum) * delb);
+        f00 = (l2 * delhu - dec) * rspan;
+        f02 = (dec - l0 * delhu) * rspan;
+        f10 = f00 * l0;
+        f11 = 0.0;
+        f12 = f02 * l2;
+    } else {  // riemann_aug_JCP, riemannsolvers.f:2-258
+        if (fabs(l1) < 1.0e-20) l1 = 0.0;
+        const double hbar = 0.5 * hsum, ghbar = g * hbar;
+        const double s1s2bar = 0.25 * (usum * usum) - ghbar;
+        const double s1s2tilde = fmax(0.0, uu) - ghbar;
+        const double rbar = rcp_near(s1s2bar);
+        const double m = (delb * g) * hbar;
+        double deldelh = div_near(m, s1s2bar, rbar);
+        const double n = ((huL - huR) + l2 * hR) - l0 * hL;
+        if (!(fmax(deldelh * l0, deldelh * l2) < n * (1.0 - 0x1p-40)))
+            deldelh = clear_bounds(deldelh, n, l0, l2);
+        double deldelphi = -div_near(m * s1s2tilde, s1s2bar, rbar);
+        const double kL = -(hL * delb), kR = -(hR * delb);
+        deldelphi = fmin(deldelphi, g * fmax(kL, kR));
+        deldelphi = fmax(deldelphi, g * fmin(kL, kR));
+        const double d0 = delh - deldelh, d2 = delphi - deldelphi;
+        const double r20 = l0 * l0, r22 = l2 * l2;
+        // det = -l2 + l0 = -(l2 - l0)
+        const double beta0 = (d0 * l2 - delhu) * rspan;
+        const double beta1 = -((((delhu * r22 - l2 * d2) - d0 * (l0 * r22 - l2 * r20)) +
+                                (l0 * d2 - delhu * r20)) * rspan);
+        const double beta2 = (delhu - d0 * l0) * rspan;
+        f00 = beta0 * l0;
+        f10 = beta0 * r20;
+        f11 = beta1;
+        f02 = beta2 * l2;
+        f12 = beta2 * r22;
+    }
+    const double f20 = f00 * vL, f22 = f02 * vR;
+    const double f21 = ((huR * vR - huL * vL) - f20) - f22;
+    const double wl = l1 < 0.0 ? 1.0 : (l1 > 0.0 ? 0.0 : 0.5), wr = 1.0 - wl;
+    const double nL1 = f10 + wl * f11, nL2 = f20 + wl * f21;
+    const double nR1 = wr * f11 + f12, nR2 = wr * f21 + f22;
+    const double s = fmax(-l0, l2);
+    fL.h = f00;
+    fL.hu = nL1 * nx - nL2 * ny;
+    fL.hv = nL1 * ny + nL2 * nx;
+    fL.s = s;
+    fR.h = f02;
+    fR.hu = nR1 * nx - nR2 * ny;
+    fR.hv = nR1 * ny + nR2 * nx;
     fR.s = s;
 }
 

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
     static_assert(!(RAW && TOL), "the toleranced kernel reads packed neighbours");
     constexpr bool GEOCLAW = SOLVER == 0 || SOLVER == 1;
     static_assert(!TOL || GEOCLAW, "toleranced GeoClaw solvers only");
-    constexpr bool CLEAR = GEOCLAW && !TOL;  // clear_flux where a wave's edges allow it
+    constexpr bool CLEAR = GEOCLAW && !TOL;  // 1/h and sqrt(g h) staged per cell
     constexpr int NW = CH / 64;
     __shared__ double s_q[4][CH];  // eta, hu, hv, b of the chunk (TOL: h, wu, wv, b)
     // CLEAR: 1/h and sqrt(g h) of each cell (clear_cell); TOL: sqrt(g h) (0 when dry)
@@ -297,14 +297,14 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         __syncthreads();
 
         __builtin_amdgcn_s_setprio(0);
-        // One pass over the list.  FIRST: a CLEAR kernel's pass with clear_flux,
+        // One pass over the list.  FIRST: a GeoClaw kernel's pass with clear_flux,
         // which leaves the rounds (of CH entries) where one of a wave's edges
         // is not clear to a second pass with the general solver; returns their
         // bits, the same for the whole wave.  A pass of its own keeps the
         // general solver's registers from adding to the shortcut's.
         auto solve = [&](auto first_pass, uint32_t rounds) -> uint32_t {
         constexpr bool FIRST = decltype(first_pass)::value;
-        constexpr bool SHORT = CLEAR && FIRST;
+        constexpr bool SHORT = GEOCLAW && FIRST;
         uint32_t rest = 0, bit = 1;
         for (int e = t; e < total; e += CH, bit <<= 1) {
             if (!FIRST && !(rounds & bit)) continue;
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
 #pragma unroll
             for (int m = 0; m < 4; ++m) L[m] = s_q[m][lc];
             if (SHORT || TOL) L[4] = s_x[0][lc];
-            if (SHORT) L[5] = s_x[CLEAR ? 1 : 0][lc];
+            if (SHORT && CLEAR) L[5] = s_x[CLEAR ? 1 : 0][lc];
             const bool inside = !(ent & LEAVES);
             const int lo = (ent >> 11) & 511;
             bool flip = false;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
 #pragma unroll
                 for (int m = 0; m < 4; ++m) R[m] = s_q[m][lo];
                 if (SHORT || TOL) R[4] = s_x[0][lo];
-                if (SHORT) R[5] = s_x[CLEAR ? 1 : 0][lo];
+                if (SHORT && CLEAR) R[5] = s_x[CLEAR ? 1 : 0][lo];
             } else if (ent & BOUNDARY) {
                 // ghost state of bnd_skeleton_scalar_op (outflow copy or mirror)
 #pragma unroll
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                     R[2] = cq.wv;
                     R[4] = cq.sq;
                 }
-                if constexpr (SHORT) {
+                if constexpr (SHORT && CLEAR) {
                     const ClearCell x = clear_cell(R[0], R[1], R[2], R[3], drytol, g);
                     R[4] = x.r;
                     R[5] = x.c;
@@ -383,19 +383,36 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 ny = flip ? -ny : ny;
             }
             Flux fL, fR;
-            if constexpr (TOL) {
-                tol::edge_flux<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], L[4], R[0], R[1], R[2], R[3],
-                                       R[4], drytol, g, inv16g, fL, fR);
-            } else if constexpr (SHORT) {
-                const double hL = L[0] - L[3], hR = R[0] - R[3];
-                const ClearEdge ce = clear_edge(nx, ny, hL, L[1], L[2], L[4], hR, R[1], R[2], R[4]);
+            if constexpr (SHORT) {
+                // normal and tangential velocities (and momenta) of both sides
+                ClearEdge ce;
+                const double hL = TOL ? L[0] : L[0] - L[3], hR = TOL ? R[0] : R[0] - R[3];
+                const double cL = TOL ? L[4] : L[5], cR = TOL ? R[4] : R[5];
+                bool clear;
+                if constexpr (TOL) {
+                    ce.uL = nx * L[1] + ny * L[2];
+                    ce.vL = nx * L[2] - ny * L[1];
+                    ce.uR = nx * R[1] + ny * R[2];
+                    ce.vR = nx * R[2] - ny * R[1];
+                    clear = tol::is_clear<SOLVER>(ce.uL, ce.uR, cL, cR);
+                } else {
+                    ce = clear_edge(nx, ny, hL, L[1], L[2], L[4], hR, R[1], R[2], R[4]);
+                    clear = is_clear<SOLVER>(ce.uL, ce.uR, cL, cR);
+                }
                 const bool dead = hL <= drytol && hR <= drytol;
-                if (__ballot(!dead && !is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5])) != 0) {
+                if (__ballot(!dead && !clear) != 0) {
                     rest |= bit;
                     continue;
                 }
-                clear_flux<SOLVER>(nx, ny, ce, hL, L[3], L[5], hR, R[3], R[5], g, fL, fR);
+                if constexpr (TOL)
+                    tol::clear_flux<SOLVER>(nx, ny, hL, ce.uL, ce.vL, L[3], cL, hR, ce.uR, ce.vR,
+                                            R[3], cR, g, fL, fR);
+                else
+                    clear_flux<SOLVER>(nx, ny, ce, hL, L[3], cL, hR, R[3], cR, g, fL, fR);
                 if (__ballot(dead) != 0 && dead) fL = fR = Flux{0.0, 0.0, 0.0, 0.0};
+            } else if constexpr (TOL) {
+                tol::edge_flux<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], L[4], R[0], R[1], R[2], R[3],
+                                       R[4], drytol, g, inv16g, fL, fR);
             } else {
                 edge_flux<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], R[0], R[1], R[2], R[3], drytol, g,
                                   inv16g, fL, fR);
@@ -416,7 +433,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         return rest;
         };
         const uint32_t rest = solve(std::true_type{}, 0u);
-        if constexpr (CLEAR) {
+        if constexpr (GEOCLAW) {
             if (rest) (void)solve(std::false_type{}, rest);
         }
         __syncthreads();

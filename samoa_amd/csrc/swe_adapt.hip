@@ -372,7 +372,7 @@ __global__ __launch_bounds__(TOP_T) void scan_top_kernel(int64_t *bsum, int64_t 
 // changes, 2: not at the fixpoint), out[3] = the last sweep that changed a
 // word, out[5] = the cells that change.  out[7] = seq goes last, a release at
 // system scope: a host that reads seq there reads the rest too.  Clears the
-// error bits for the next count pass.
+// error bits for the next count pass and the emit's count of raster cells.
 __global__ __launch_bounds__(TOP_T) void plan_top_kernel(int64_t *bsum, int64_t nb,
                                                          uint32_t *status, const int64_t *res,
                                                          int64_t *out, int64_t seq) {
@@ -385,6 +385,7 @@ __global__ __launch_bounds__(TOP_T) void plan_top_kernel(int64_t *bsum, int64_t 
         out[3] = (int64_t)status[1];
         out[5] = total >> 32;
         status[0] = 0u;
+        status[2] = 0u;  // raster_count of the emit that may follow
         __hip_atomic_store(&out[7], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
@@ -634,46 +635,85 @@ __device__ double raster_sample(const AdaptArgs &a, double X, double Y) {
            wx * wy * r1[1];
 }
 
-// b of a new cell of corners c and depth d from the raster, as
-// get_bathymetry_at_element computes it under _ADAPT_INTEGRATE
-// (SWE_initialize.f90:106-147) for gridded data: L = min(16, raster_cap - d)
-// halvings of the cell (raster_cap = min(dmax + 3, data_depth + 3)), each
-// level 0.5 (value of the first half (x1, m, x2) + value of the second
-// (x2, m, x3)), the raster at the centroid scaling * (x1 + x2 + x3) / 3 +
-// offset at the bottom; L <= 0 is that centroid sample alone.  The 2^L
-// leaves run in depth-first order, a leaf's corners found by L halvings
-// along its index; a stack of partial values combines each finished pair as
-// the recursion does.
-__device__ double raster_cell(const AdaptArgs &a, const double c[6], int d) {
-    const int levels = min(16, a.raster_cap - d);
-    if (levels <= 0) {  // a cell finer than the data: its centroid (no stack)
-        const double cx = (c[0] + c[2] + c[4]) / 3.0, cy = (c[1] + c[3] + c[5]) / 3.0;
-        return raster_sample(a, a.scaling * cx + a.offset_x, a.scaling * cy + a.offset_y);
+// One halving of the cell c: its second child (x2, m, x3) or its first
+// (x1, m, x2), m = 0.5 (x1 + x3).
+__device__ __forceinline__ void halve(double c[6], bool second) {
+    const double mx = 0.5 * (c[0] + c[4]), my = 0.5 * (c[1] + c[5]);
+    if (second) {
+        c[0] = c[2];
+        c[1] = c[3];
+    } else {
+        c[4] = c[2];
+        c[5] = c[3];
     }
-    double stack[17];
+    c[2] = mx;
+    c[3] = my;
+}
+
+// The raster at the centroid of a cell.
+__device__ __forceinline__ double raster_centroid(const AdaptArgs &a, const double c[6]) {
+    const double cx = (c[0] + c[2] + c[4]) / 3.0, cy = (c[1] + c[3] + c[5]) / 3.0;
+    return raster_sample(a, a.scaling * cx + a.offset_x, a.scaling * cy + a.offset_y);
+}
+
+// Halvings of a new cell at depth d under get_bathymetry_at_element's
+// _ADAPT_INTEGRATE rule for gridded data (SWE_initialize.f90:106-147):
+// min(16, raster_cap - d), raster_cap = min(dmax + 3, data_depth + 3); none
+// is the centroid sample alone.
+__device__ __forceinline__ int raster_levels(const AdaptArgs &a, int d) {
+    return max(0, min(16, a.raster_cap - d));
+}
+
+// b of a cell of corners c over `levels` halvings: each level 0.5 (value of
+// the first half + value of the second), the raster at the centroid at the
+// bottom.  The leaves run in depth-first order, two levels of them at once
+// (their samples are independent); a stack of partial values combines each
+// finished pair as the recursion does.
+__device__ double raster_serial(const AdaptArgs &a, const double c[6], int levels) {
+    if (levels <= 0) return raster_centroid(a, c);
+    const int tail = levels < 2 ? levels : 2;  // levels below a block of leaves
+    const int blocks = 1 << (levels - tail);
+    double stack[15];
     int sp = 0;
-    const int leaves = levels > 0 ? 1 << levels : 1;
-    for (int i = 0; i < leaves; ++i) {
-        double ax = c[0], ay = c[1], bx = c[2], by = c[3], ex = c[4], ey = c[5];
-        for (int l = levels - 1; l >= 0; --l) {
-            const double mx = 0.5 * (ax + ex), my = 0.5 * (ay + ey);
-            if ((i >> l) & 1) {  // (x2, m, x3)
-                ax = bx;
-                ay = by;
-            } else {  // (x1, m, x2)
-                ex = bx;
-                ey = by;
-            }
-            bx = mx;
-            by = my;
+    for (int i = 0; i < blocks; ++i) {
+        double q[6] = {c[0], c[1], c[2], c[3], c[4], c[5]};
+        for (int l = levels - tail - 1; l >= 0; --l) halve(q, (i >> l) & 1);
+        double v4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            double r[6] = {q[0], q[1], q[2], q[3], q[4], q[5]};
+            if (tail == 2) halve(r, j >> 1);
+            halve(r, j & 1);
+            v4[j] = tail == 2 || j < 2 ? raster_centroid(a, r) : 0.0;
         }
-        const double cx = (ax + bx + ex) / 3.0, cy = (ay + by + ey) / 3.0;
-        double v = raster_sample(a, a.scaling * cx + a.offset_x, a.scaling * cy + a.offset_y);
+        double v = 0.5 * (v4[0] + v4[1]);
+        if (tail == 2) v = 0.5 * (v + 0.5 * (v4[2] + v4[3]));
         for (int j = i; j & 1; j >>= 1) v = 0.5 * (stack[--sp] + v);
         stack[sp++] = v;
     }
     return stack[0];
 }
+
+// The same by a whole wave (every lane gets the value): each lane takes the
+// part of the tree that its number spells, then the parts combine pairwise,
+// 0.5 (first + second) at every level as above.
+__device__ double raster_wave(const AdaptArgs &a, const double c[6], int levels) {
+    const int lane = threadIdx.x & 63, top = levels < 6 ? levels : 6;
+    double q[6] = {c[0], c[1], c[2], c[3], c[4], c[5]};
+    for (int l = top - 1; l >= 0; --l) halve(q, (lane >> l) & 1);
+    double v = raster_serial(a, q, levels - top);
+    for (int l = 0; l < top; ++l) v = 0.5 * (v + __shfl_xor(v, 1 << l, 64));
+    return v;
+}
+
+// A new cell of more halvings than this leaves its b to raster_kernel: a
+// child at depth 11 of a depth-18 run averages 1024 samples, a serial chain of
+// gathers that held one thread, and the emit with it, for 3.1-3.8 ms of every
+// changing remeshing; a wave per child takes 6-15 us.  Two samples at most
+// are cheaper in the emit's thread than in a kernel of their own (a deep run,
+// depths 16-26, has mostly one, and pays the 5 us of that kernel where a
+// coarse cell may split).
+constexpr int RASTER_INLINE = 1;
 
 __device__ __forceinline__ void put_slot(int32_t *eslot, int64_t c, int k, int half, int32_t v) {
     if (half == 2) {
@@ -682,14 +722,6 @@ __device__ __forceinline__ void put_slot(int32_t *eslot, int64_t c, int k, int h
     } else {
         eslot[6 * c + 2 * k + half] = v;
     }
-}
-
-// The new cell-edge on half s of old edge k of cell c: computed for a cell
-// that keeps its place, read from the slots emit_change_kernel wrote otherwise.
-__device__ __forceinline__ int32_t edge_slot(const AdaptArgs &a, int64_t c, int k, int s) {
-    const int32_t kc = a.kidx[c];
-    if (kc >= 0) return (kc << 2) | k;
-    return a.eslot[6 * c + 2 * k + s];
 }
 
 // The cells that keep their place: a shifted copy of depth, plotter type,
@@ -781,6 +813,7 @@ __global__ __launch_bounds__(CHANGE_T) void emit_change_kernel(AdaptArgs a) {
         int64_t coff = off0;  // tree offset of the next child
         double pc[6];         // the parent's corners, for the raster
         if (a.raster) tree_corners(coff, 0, d, pc);
+        bool later = false;
         for (int j = 0; j < cells; ++j) {
             const uint64_t w = j == 0 ? w0 : j == 1 ? w1 : j == 2 ? w2 : w3;
             const int rule = (int)((w >> 8) & 0xff);
@@ -800,7 +833,9 @@ __global__ __launch_bounds__(CHANGE_T) void emit_change_kernel(AdaptArgs a) {
             if (a.raster) {
                 double cc[6] = {pc[0], pc[1], pc[2], pc[3], pc[4], pc[5]};
                 tree_corners(coff, d, dc, cc);
-                a.b_out[idx] = raster_cell(a, cc, dc);
+                const int levels = raster_levels(a, dc);
+                if (a.raster_list && levels > RASTER_INLINE) later = true;
+                else a.b_out[idx] = raster_serial(a, cc, levels);
             } else {
                 a.b_out[idx] = bc;
             }
@@ -814,6 +849,28 @@ __global__ __launch_bounds__(CHANGE_T) void emit_change_kernel(AdaptArgs a) {
                 }
             }
         }
+        if (later) a.raster_list[atomicAdd(a.raster_count, 1u)] = (uint32_t)c;
+    }
+}
+
+// b of the children that emit_change_kernel left (raster_list: their split
+// cells, in any order): a workgroup per split cell, a wave per child.
+constexpr int RASTER_T = 256, RASTER_BLOCKS = 2048;
+__global__ __launch_bounds__(RASTER_T) void raster_kernel(AdaptArgs a) {
+    const uint32_t count = *a.raster_count;
+    const int j = threadIdx.x >> 6;  // the child
+    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+        const int64_t c = a.raster_list[i];
+        const int pat = a.code[c] - CODE_SPLIT;
+        if (j >= 2 + (pat & 1) + (pat >> 1)) continue;
+        const int64_t idx = (a.base[c] & 0xffffffffLL) + j;
+        const int dc = a.depth_out[idx];
+        const int levels = raster_levels(a, dc);
+        if (levels <= RASTER_INLINE) continue;  // written by emit_change_kernel
+        double q[6];
+        tree_corners(a.off_out[idx], 0, dc, q);
+        const double v = raster_wave(a, q, levels);
+        if ((threadIdx.x & 63) == 0) a.b_out[idx] = v;
     }
 }
 
@@ -1086,8 +1143,15 @@ hipError_t identity_record(int64_t n, int8_t *code, int64_t *base, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t adapt_emit(const AdaptArgs &a, hipStream_t s, bool prefix_done) {
+hipError_t adapt_emit(const AdaptArgs &args, hipStream_t s, bool prefix_done) {
+    AdaptArgs a = args;
     const int64_t tiles = adapt_scan_tiles(a.n);
+    // the children of a mesh at its depth range: with few halvings each, the
+    // emit samples them itself
+    if (a.raster && a.raster_cap - (a.dmin + 1) > RASTER_INLINE) {
+        a.raster_list = a.slots;  // the conformity words are not read any more
+        a.raster_count = a.status + 2;
+    }
     if (tiles > 0 && !prefix_done)
         scan_codes_kernel<<<(unsigned)tiles, SCAN_T, 0, s>>>(a.n, a.code, a.bsum, a.base, a.kidx,
                                                              a.list);
@@ -1096,6 +1160,9 @@ hipError_t adapt_emit(const AdaptArgs &a, hipStream_t s, bool prefix_done) {
     if (e != hipSuccess || a.n_changing == 0) return e;
     emit_change_kernel<<<blocks_for(a.n_changing, CHANGE_T), CHANGE_T, 0, s>>>(a);
     link_kernel<<<blocks_for(a.n_changing, CHANGE_T), CHANGE_T, 0, s>>>(a);
+    if (a.raster_list)
+        raster_kernel<<<(unsigned)(a.n_changing < RASTER_BLOCKS ? a.n_changing : RASTER_BLOCKS),
+                        RASTER_T, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -130,6 +130,9 @@ struct AdaptArgs {
     // a new cell at depth d averages the raster over min(16, raster_cap - d)
     // halvings (_ADAPT_INTEGRATE); raster_cap = min(dmax + 3, data_depth + 3)
     int raster_cap;
+    // split cells whose children's b a kernel after the emit samples, and
+    // their number (set by adapt_emit; null: the emit samples every child)
+    uint32_t *raster_list, *raster_count;
 };
 
 // bsum holds adapt_scan_tiles(n) + 1 scan words and 8 result words.

@@ -133,8 +133,8 @@ int ensure_tables(int device) {
 // would otherwise capture again.
 struct GraphCache {
     hipGraphExec_t exec = nullptr;
-    int cur = -1, forward = -1, chunk = 0, keep = -1, jumps = -1, tol = -1;
-    double jump_refine = 0.0, jump_coarsen = 0.0;
+    int cur = -1, forward = -1, chunk = 0, keep = -1, jumps = -1, tol = -1, pp = -1;
+    double jump_refine = 0.0, jump_coarsen = 0.0, dt_clamp = 0.0;
     int64_t grid = -1;
 };
 
@@ -211,8 +211,14 @@ struct Batch {
     int32_t *d_chunk_scen = nullptr;
     swe::Slots *d_slots = nullptr;
     double *d_dt = nullptr;  // [nscen] host-chosen dt per scenario
-    double *d_part_min = nullptr;     // [part_cap] CFL minimum per chunk
+    double *d_part_max[2] = {nullptr, nullptr};  // [part_cap] fastest cell per chunk
     int32_t *d_part_nref = nullptr;   // [part_cap] refinement count per chunk
+    // A chain of steps without finalize kernels (batch_run): the device dt is
+    // not in the slots yet, but in the partials of the last step,
+    // d_part_max[pp], over the pend_chunks chunks that mesh had.
+    bool pending = false;
+    int pp = 0;
+    int64_t pend_chunks = 0;
     int64_t part_cap = 0;
     double *eta[2] = {nullptr, nullptr}, *hu[2] = {nullptr, nullptr}, *hv[2] = {nullptr, nullptr};
     double *b = nullptr;
@@ -284,7 +290,8 @@ void release(Batch &B) {
     (void)hipFree(B.d_chunk_scen);
     (void)hipFree(B.d_slots);
     (void)hipFree(B.d_dt);
-    (void)hipFree(B.d_part_min);
+    (void)hipFree(B.d_part_max[0]);
+    (void)hipFree(B.d_part_max[1]);
     (void)hipFree(B.d_part_nref);
     (void)hipFree(B.b2);
     (void)hipFree(B.nbr2);
@@ -309,6 +316,21 @@ bool all_uploaded(const Batch &B) {
     return std::all_of(B.uploaded.begin(), B.uploaded.end(), [](char c) { return c != 0; });
 }
 
+swe::StepArgs make_args(const Batch &B, int from, int to, int forward);
+
+// Brings the device dt of a chain of steps into the slots.
+int chain_flush(Batch &B) {
+    if (!B.pending) return SWE_OK;
+    swe::StepArgs a = make_args(B, 0, 1, 0);
+    a.part_max = B.d_part_max[B.pp];
+    a.device_dt = 1;
+    a.chained = 1;
+    a.prev_chunks = (int32_t)B.pend_chunks;
+    HIP_TRY(swe::launch_finalize(a, B.stream));
+    B.pending = false;
+    return SWE_OK;
+}
+
 // Chunk tables for the current chunk size: chunk offsets per scenario and the
 // chunk -> scenario map (not needed for a single scenario).
 // upload = false: the device copy of the scenario table is already
@@ -325,13 +347,16 @@ int rebuild_chunks(Batch &B, bool upload = true) {
         return fail(SWE_ERR_ARG, "too many chunks (%lld)", (long long)B.nchunks);
     if (B.nchunks > B.part_cap) {  // with room to grow: remeshing changes the count
         const int64_t cap = B.nchunks + B.nchunks / 4;
+        SWE_TRY(chain_flush(B));
         if (B.stream) HIP_TRY(hipStreamSynchronize(B.stream));
-        (void)hipFree(B.d_part_min);
+        (void)hipFree(B.d_part_max[0]);
+        (void)hipFree(B.d_part_max[1]);
         (void)hipFree(B.d_part_nref);
-        B.d_part_min = nullptr;
+        B.d_part_max[0] = B.d_part_max[1] = nullptr;
         B.d_part_nref = nullptr;
         B.part_cap = 0;
-        if (hipMalloc(&B.d_part_min, sizeof(double) * (size_t)cap) != hipSuccess ||
+        if (hipMalloc(&B.d_part_max[0], sizeof(double) * (size_t)cap) != hipSuccess ||
+            hipMalloc(&B.d_part_max[1], sizeof(double) * (size_t)cap) != hipSuccess ||
             hipMalloc(&B.d_part_nref, sizeof(int32_t) * (size_t)cap) != hipSuccess)
             return fail(SWE_ERR_NOMEM, "chunk partials allocation failed");
         B.part_cap = cap;
@@ -477,7 +502,7 @@ swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
     a.scen0 = B.scen[0];  // read in place of the table when it is the only one
     a.chunk_scen = B.d_chunk_scen;
     a.slots = B.d_slots;
-    a.part_min = B.d_part_min;
+    a.part_max = B.d_part_max[1 - B.pp];  // not the one a chain may still need
     a.part_nref = B.d_part_nref;
     a.n_scen = B.nscen;
     a.nchunks = B.nchunks;
@@ -556,14 +581,17 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     if (n_steps < 0 || (dt0 && !time)) return fail(SWE_ERR_ARG, "run: invalid argument");
     if (!all_uploaded(B)) return fail(SWE_ERR_STATE, "run: not every scenario has a state");
     bool table_changed = false;
-    for (auto &s : B.scen)
-        if (s.dt_clamp != dt_clamp) {
-            s.dt_clamp = dt_clamp;
-            table_changed = true;
-        }
-    if (table_changed)
+    for (auto &s : B.scen) table_changed |= s.dt_clamp != dt_clamp;
+    if (dt0) {
+        B.pending = false;  // the chain starts again
+    } else if (table_changed) {
+        SWE_TRY(chain_flush(B));  // the dt the last run left is clamped as that run was
+    }
+    if (table_changed) {
+        for (auto &s : B.scen) s.dt_clamp = dt_clamp;
         HIP_TRY(hipMemcpyAsync(B.d_scen, B.scen.data(), sizeof(swe::Scen) * B.scen.size(),
                                hipMemcpyHostToDevice, B.stream));
+    }
     // the chain starts from dt0 (clamped as pre_traversal_grid_op does) and the
     // caller's time
     if (dt0) {
@@ -576,19 +604,51 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
                                hipMemcpyHostToDevice, B.stream));
     }
 
-    auto one_step = [&](hipStream_t st, int from, int fwd) -> hipError_t {
+    // Meshes of few chunks step in a chain: a step forms its dt from the
+    // partials of the one before, and a finalize kernel runs only for who
+    // reads the results.
+    bool chain = true;
+    for (auto &s : B.scen) chain = chain && s.nchunks <= swe::CHAIN_CHUNKS;
+    if (!chain) SWE_TRY(chain_flush(B));
+    // one step from state buffer `from`; in a chain, with the partials
+    // d_part_max[pp] of the step before if there is one
+    auto one_step = [&](hipStream_t st, int from, int fwd, bool prev, int pp) -> hipError_t {
         swe::StepArgs a = make_args(B, from, 1 - from, fwd);
         a.device_dt = 1;
         a.refine = B.keep_flags ? B.refine : nullptr;
+        if (chain) {
+            a.chained = 1;
+            a.skip_finalize = 1;
+            a.part_max = B.d_part_max[1 - pp];
+            a.prev_max = prev ? B.d_part_max[pp] : nullptr;
+            a.prev_chunks = (int32_t)B.pend_chunks;
+        }
         return swe::launch_step(a, B.solver, B.chunk, B.grid, st);
     };
     int fwd = forward ? 1 : 0;
-    const int64_t pairs = n_steps / 2;
+    int64_t left = n_steps;
+    auto single = [&]() -> int {
+        HIP_TRY(one_step(B.stream, B.cur, fwd, B.pending, B.pp));
+        B.cur = 1 - B.cur;
+        fwd = 1 - fwd;
+        --left;
+        if (chain) {
+            B.pending = true;
+            B.pp = 1 - B.pp;
+            B.pend_chunks = B.nchunks;
+        }
+        return SWE_OK;
+    };
+    // the first step of a chain, and the first after a remeshing, reads its
+    // dt from elsewhere than the captured ones
+    if (chain && left > 0 && (!B.pending || B.pend_chunks != B.nchunks)) SWE_TRY(single());
+    const int64_t pairs = left / 2;
     if (pairs > 0) {
         GraphCache &gc = B.graph[B.cur][fwd];
+        const int pp = chain ? B.pp : -1;
         if (!gc.exec || gc.cur != B.cur || gc.forward != fwd || gc.chunk != B.chunk ||
             gc.grid != B.grid || gc.keep != B.keep_flags || gc.jumps != B.jump_flags ||
-            gc.tol != B.tol ||
+            gc.tol != B.tol || gc.pp != pp || gc.dt_clamp != dt_clamp ||
             gc.jump_refine != B.jump_refine || gc.jump_coarsen != B.jump_coarsen) {
             if (gc.exec) {
                 (void)hipGraphExecDestroy(gc.exec);
@@ -598,8 +658,9 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
             HIP_TRY(hipStreamSynchronize(B.stream));
             hipGraph_t graph;
             HIP_TRY(hipStreamBeginCapture(B.own_stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e1 = one_step(B.own_stream, B.cur, fwd);
-            hipError_t e2 = e1 == hipSuccess ? one_step(B.own_stream, 1 - B.cur, 1 - fwd) : e1;
+            hipError_t e1 = one_step(B.own_stream, B.cur, fwd, true, B.pp);
+            hipError_t e2 =
+                e1 == hipSuccess ? one_step(B.own_stream, 1 - B.cur, 1 - fwd, true, 1 - B.pp) : e1;
             hipError_t e3 = hipStreamEndCapture(B.own_stream, &graph);
             if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess)
                 return fail(SWE_ERR_HIP, "run: graph capture failed: %s",
@@ -614,17 +675,18 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
             gc.keep = B.keep_flags;
             gc.jumps = B.jump_flags;
             gc.tol = B.tol;
+            gc.pp = pp;
+            gc.dt_clamp = dt_clamp;
             gc.jump_refine = B.jump_refine;
             gc.jump_coarsen = B.jump_coarsen;
         }
         for (int64_t i = 0; i < pairs; ++i) HIP_TRY(hipGraphLaunch(gc.exec, B.stream));
+        left -= 2 * pairs;
     }
-    if (n_steps % 2) {
-        HIP_TRY(one_step(B.stream, B.cur, fwd));
-        B.cur = 1 - B.cur;
-    }
+    if (left > 0) SWE_TRY(single());
     if (n_steps > 0) B.flags_valid = B.keep_flags != 0;
     if (!time && !dt_next) return SWE_OK;
+    SWE_TRY(chain_flush(B));
     std::vector<swe::Slots> res((size_t)B.nscen);
     HIP_TRY(hipMemcpyAsync(res.data(), B.d_slots, sizeof(swe::Slots) * res.size(),
                            hipMemcpyDeviceToHost, B.stream));
@@ -1010,6 +1072,7 @@ int batch_set_tuning(Batch &B, int chunk, int64_t grid) {
     if (!known) return fail(SWE_ERR_ARG, "chunk size %d not compiled (128, 256 or 512)", chunk);
     if (grid < 0 || grid % 8) return fail(SWE_ERR_ARG, "grid %lld must be 0 or a multiple of 8", (long long)grid);
     HIP_TRY(hipStreamSynchronize(B.stream));
+    SWE_TRY(chain_flush(B));
     B.grid = grid;
     if (chunk != B.chunk) {
         B.chunk = chunk;
@@ -1367,7 +1430,7 @@ int swe_step_device_noalloc(const swe_device_mesh *m, const double *eta, const d
     a.depth = m->depth;
     a.refine = refine_dev;
     a.slots = (swe::Slots *)scr;
-    a.part_min = (double *)(scr + NOALLOC_SLOT_BYTES);
+    a.part_max = (double *)(scr + NOALLOC_SLOT_BYTES);
     a.part_nref = (int32_t *)(scr + NOALLOC_SLOT_BYTES + sizeof(double) * NOALLOC_MAX_CHUNKS);
     a.out_dtcfl = dt_cfl_dev;
     a.out_nref = n_refine_dev;

@@ -12,9 +12,10 @@ namespace swe {
 constexpr int CHUNK_SIZES[3] = {128, 256, 512};
 constexpr int DEFAULT_CHUNK = 256;
 
-// Per-scenario results and device dt chain.  Written only by the finalize
-// kernel that follows each step kernel on the stream; the step kernel reads
-// dt.
+// Per-scenario results and device dt chain.  The finalize kernel that follows
+// a step kernel on the stream writes them; the step kernel reads dt.  Steps
+// in a chain (StepArgs::chained) run without a finalize kernel between them:
+// each advances time, and the one after it forms its dt from the partials.
 struct Slots {
     double dt;                   // dt of the next step (device dt chain)
     double time;                 // simulated time (device dt chain)
@@ -51,7 +52,9 @@ struct StepArgs {
     const double *dt_host;                 // [n_scen] dt per scenario when device_dt == 0, or null
     double *out_dtcfl;                     // [n_scen] extra copy of the CFL minima, or null
     int64_t *out_nref;                     // [n_scen] extra copy of the refinement counts, or null
-    double *part_min;                      // [nchunks] CFL minimum of each chunk
+    // [nchunks] largest sv 2^(d+1) of each chunk (its CFL minimum is S^2
+    // divided by it), 0 without a limit
+    double *part_max;
     int32_t *part_nref;                    // [nchunks] refinement count of each chunk
     int32_t n_scen;
     int64_t nchunks;
@@ -59,7 +62,14 @@ struct StepArgs {
     double g, inv16g;                      // inv16g = 1 / (16 g), riemannsolvers.f:556
     int bc, forward;
     int device_dt;                         // 1: read dt from slots[s].dt and write the next one
-    int skip_finalize;                     // 1: nobody reads this step's CFL results
+    int skip_finalize;                     // 1: no finalize kernel after this step
+    // Chains of steps with device_dt: chained != 0: this step adds its dt to
+    // slots[s].time itself.  prev_max: the last step's part_max (then dt comes
+    // from it instead of slots[s].dt), prev_chunks its chunks when there is
+    // one scenario (a remeshing may have changed them since).
+    int chained;
+    int32_t prev_chunks;
+    const double *prev_max;
     // refinement flags from surface-elevation jumps between wet neighbours
     // of the state the step reads (refine above jump_refine, coarsen below
     // jump_coarsen) instead of volume_op's |dQ_h| criterion
@@ -189,6 +199,14 @@ hipError_t launch_adjoint(const AdjArgs &a, int solver, int chunk, int64_t grid_
 // grid_blocks: number of workgroups (multiple of 8) or 0 for one per chunk.
 hipError_t launch_step(const StepArgs &a, int solver, int chunk, int64_t grid_blocks,
                        hipStream_t s);
+// The finalize kernel alone, after a chain of steps (a.chained).
+hipError_t launch_finalize(const StepArgs &a, hipStream_t s);
+// Largest number of chunks per scenario for which a step forms its dt from
+// the partials of the step before.  Every workgroup reads all of them, so a
+// chain trades the finalize kernel (4-5 us with its launch) for nchunks^2
+// reads from L2.  100 steps: 1.33 -> 1.06 ms at 128 chunks, 2.81 -> 2.39 at
+// 1024, 4.24 -> 4.11 at 2048, but 6.75 -> 7.56 at 4096.
+constexpr int64_t CHAIN_CHUNKS = 2048;
 // The step of a single mesh whose nbr holds plain neighbour cells
 // (StepArgs::raw_nbr), chunk DEFAULT_CHUNK, one workgroup per chunk, flags
 // by volume_op's criterion; then the finalize kernel.

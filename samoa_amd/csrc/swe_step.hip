@@ -50,12 +50,6 @@ namespace swe {
 __constant__ double c_normal[17 * 3 * 2];  // [plotter + 8][edge][x,y]
 __constant__ double c_leg[64];             // l(k) = sqrt(0.5)**k at k + 1
 
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = dmin2(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // A pointer to memory that no kernel writes while this one runs, for scalar
 // loads from uniform addresses.
 template <typename T>
@@ -70,8 +64,8 @@ __device__ __forceinline__ double max_f64(double a, double b) {
     return r;
 }
 
-// Lane 63 gets the maximum of values >= 0 over the wave (NaN only if every
-// value is one): row shifts by 1, 2, 4 and 8, then the rows' last lanes
+// Lane 63 gets the maximum over the wave of values >= 0 (0 without any; NaN
+// values are left out): row shifts by 1, 2, 4 and 8, then the rows' last lanes
 // broadcast to the next row and half; a lane without a source reads 0.
 __device__ __forceinline__ double wave_max(double v) {
     auto step = [&](auto ctrl) {
@@ -87,6 +81,17 @@ __device__ __forceinline__ double wave_max(double v) {
     step(std::integral_constant<int, 0x142>{});
     step(std::integral_constant<int, 0x143>{});
     return v;
+}
+
+// The CFL minimum (huge(1.0_SR) without a limit, pre_traversal_op :139) from
+// the largest sv 2^(d+1), and the dt it gives (post_traversal_grid_op
+// :117-118, pre_traversal_grid_op :93-99).
+__device__ __forceinline__ double cfl_minimum(double scaling, double fastest) {
+    return dmin2(1.7976931348623157e308, (scaling * scaling) / fastest);
+}
+__device__ __forceinline__ double next_dt(double courant, double dt_clamp, double dt_cfl) {
+    const double next = courant * dt_cfl;
+    return dt_clamp > 0.0 ? dmin2(dt_clamp, next) : next;
 }
 
 // Lanes of the mask below this one.
@@ -129,7 +134,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
     __shared__ uint32_t s_list[3 * CH + 4];
     __shared__ uint32_t s_jb[JUMPS ? CH / 16 : 1];  // elevation-jump bits, 2 per cell
     __shared__ int s_wsum[NW];
-    __shared__ double s_wmax[NW];
+    __shared__ double s_wmax[NW], s_dt;
     __shared__ int s_wref[NW];
     // geometry tables in LDS: the per-lane indexed reads would otherwise be
     // global loads that every edge waits for
@@ -188,9 +193,18 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         const int8_t *const c_plot = a.plotter + gt + lbase;
         const int8_t *const c_depth = a.depth + gt + lbase;
         const int64_t c_out = gs + lbase;  // first output cell of the chunk
-        const double dt = a.device_dt ? scalar(a.slots)[s].dt
-                                      : (a.dt_host ? scalar(a.dt_host)[s] : a.dt);
+        double dt = a.device_dt ? scalar(a.slots)[s].dt
+                                : (a.dt_host ? scalar(a.dt_host)[s] : a.dt);
         const double drytol = sc.drytol;
+
+        // a chain: the last step's fastest cell, from its chunks' partials
+        // (the minimum waits for the loads only after the staging's)
+        double fastest = 0.0;
+        if (!RAW && a.prev_max) {
+            const int n = a.chunk_scen ? (int)sc.nchunks : a.prev_chunks;
+            const double *const pm = a.prev_max + (a.chunk_scen ? sc.chunk_off : 0);
+            for (int i0 = t; i0 < n; i0 += CH) fastest = max_f64(fastest, pm[i0]);
+        }
 
         int32_t nb[3] = {-1, -1, -1};
         int plot = 1;
@@ -262,7 +276,17 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         if (lane == 0)
             s_wsum[wave] = __popcll(i0) + 2 * __popcll(i1) +
                            ((__popcll(o0) + 2 * __popcll(o1)) << 16);
+        if (!RAW && a.prev_max) {
+            const double w = wave_max(fastest);
+            if (lane == 63) s_wmax[wave] = w;
+        }
         __syncthreads();
+        if (!RAW && a.prev_max && t == 0) {
+            double m = s_wmax[0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) m = max_f64(m, s_wmax[w]);
+            s_dt = next_dt(sc.courant, sc.dt_clamp, cfl_minimum(sc.scaling, m));
+        }
         int pre = wpre, sum = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
@@ -439,11 +463,12 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         __syncthreads();
 
         // cell update: volume_op + cell_update_op
+        if (!RAW && a.prev_max) dt = s_dt;
+        if (a.chained && lbase == 0 && t == 0) a.slots[s].time = a.slots[s].time + dt;
         // The CFL candidate of a cell is fl(volume / sv), volume = S^2 2^-(d+1):
         // scaling by a power of two is exact and the rounded quotient falls
-        // as the divisor grows, so the chunk's minimum is the quotient of S^2
-        // and the largest sv 2^(d+1) (without cells: huge(1.0_SR),
-        // pre_traversal_op :139)
+        // as the divisor grows, so a mesh's minimum is the quotient of S^2
+        // and the largest sv 2^(d+1) (a cell whose sv is NaN has no limit).
         double speed = 0.0;
         bool refined = false;
         if (active) {
@@ -539,7 +564,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 m = max_f64(m, s_wmax[w]);
                 rsum += s_wref[w];
             }
-            a.part_min[chunk] = (sc.scaling * sc.scaling) / m;
+            a.part_max[chunk] = m;
             a.part_nref[chunk] = rsum;
         }
         __syncthreads();  // LDS is reused by the next chunk
@@ -560,19 +585,19 @@ constexpr int FIN_THREADS = 1024;
 // chunks.
 constexpr int FIN_PER = 16;
 __global__ __launch_bounds__(FIN_THREADS) void finalize_kernel(StepArgs a) {
-    __shared__ double s_min[FIN_THREADS / 64];
+    __shared__ double s_max[FIN_THREADS / 64];
     __shared__ long long s_ref[FIN_THREADS / 64];
     const int s = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const Scen sc = a.scen ? a.scen[s] : a.scen0;
     Slots *sl = &a.slots[s];
     const double time0 = sl->time, dt0 = sl->dt;  // every thread: no branch to wait at
-    const double huge = 1.7976931348623157e308;  // huge(1.0_SR)
-    double m = huge;
+    double m = 0.0;
     long long r = 0;
-    const double *pm = a.part_min + sc.chunk_off;
+    const double *pm = a.part_max + sc.chunk_off;
     const int32_t *pr = a.part_nref + sc.chunk_off;
-    const int64_t nc = sc.nchunks;
+    // the chunks of the chain's last step, if a remeshing came after it
+    const int64_t nc = a.chained && a.n_scen == 1 ? a.prev_chunks : sc.nchunks;
     for (int64_t i0 = t; i0 < nc; i0 += (int64_t)FIN_PER * FIN_THREADS) {
         double v[FIN_PER];
         int32_t w[FIN_PER];
@@ -586,35 +611,34 @@ __global__ __launch_bounds__(FIN_THREADS) void finalize_kernel(StepArgs a) {
 #pragma unroll
         for (int j = 0; j < FIN_PER; ++j) {
             const bool in = i0 + (int64_t)j * FIN_THREADS < nc;
-            m = dmin2(m, in ? v[j] : huge);
+            m = max_f64(m, in ? v[j] : 0.0);
             r += in ? w[j] : 0;
         }
     }
-    m = wave_min(m);
+    m = wave_max(m);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off, 64);
-    if (lane == 0) {
-        s_min[wave] = m;
+    if (lane == 63) {
+        s_max[wave] = m;
         s_ref[wave] = r;
     }
     __syncthreads();
     if (t == 0) {
-        m = s_min[0];
+        m = s_max[0];
         r = s_ref[0];
 #pragma unroll
         for (int w = 1; w < FIN_THREADS / 64; ++w) {
-            m = dmin2(m, s_min[w]);
+            m = max_f64(m, s_max[w]);
             r += s_ref[w];
         }
+        m = cfl_minimum(sc.scaling, m);
         sl->res_dtcfl = m;
         sl->res_nref = r;
         if (a.out_dtcfl) a.out_dtcfl[s] = m;
         if (a.out_nref) a.out_nref[s] = (int64_t)r;
         if (a.device_dt) {
-            sl->time = time0 + dt0;
-            double next = sc.courant * m;
-            if (sc.dt_clamp > 0.0) next = dmin2(sc.dt_clamp, next);
-            sl->dt = next;
+            if (!a.chained) sl->time = time0 + dt0;
+            sl->dt = next_dt(sc.courant, sc.dt_clamp, m);
         }
     }
 }
@@ -623,6 +647,11 @@ hipError_t upload_tables(const double *normal, const double *leg) {
     hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_normal), normal, sizeof(double) * 17 * 3 * 2);
     if (e != hipSuccess) return e;
     return hipMemcpyToSymbol(HIP_SYMBOL(c_leg), leg, sizeof(double) * 64);
+}
+
+hipError_t launch_finalize(const StepArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)a.n_scen), dim3(FIN_THREADS), 0, s, a);
+    return hipGetLastError();
 }
 
 template <int SOLVER, int CH>

@@ -26,6 +26,8 @@
 // each XCD's L2 holds the halos of its own chunks; a grid smaller than the
 // chunk count makes the launch persistent (grid-stride).
 //
+// NT threads work on a chunk, CH or 2 CH; the first CH hold a cell each.
+//
 // Edge semantics (Tools_adaptive_traversal.f90:606-640).  The left state of
 // an interior edge is the cell that touches it first in the current
 // traversal direction: the lower SFC index when forward, the higher when
@@ -113,14 +115,14 @@ constexpr uint32_t LEAVES = 1u << 31, BOUNDARY = 1u << 30;
 // solvers only): the chunk stages each cell's depth, world velocity,
 // bathymetry and sqrt(g h) instead of its state and keeps its own state in
 // registers.
-template <int SOLVER, int CH, bool JUMPS, bool RAW = false, bool TOL = false>
-__global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void euler_step_kernel(
+template <int SOLVER, int CH, int NT, bool JUMPS, bool RAW = false, bool TOL = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void euler_step_kernel(
     StepArgs args) {
     static_assert(!(RAW && TOL), "the toleranced kernel reads packed neighbours");
     constexpr bool GEOCLAW = SOLVER == 0 || SOLVER == 1;
     static_assert(!TOL || GEOCLAW, "toleranced GeoClaw solvers only");
     constexpr bool CLEAR = GEOCLAW && !TOL;  // 1/h and sqrt(g h) staged per cell
-    constexpr int NW = CH / 64;
+    constexpr int NW = NT / 64;
     __shared__ double s_q[4][CH];  // eta, hu, hv, b of the chunk (TOL: h, wu, wv, b)
     // CLEAR: 1/h and sqrt(g h) of each cell (clear_cell); TOL: sqrt(g h) (0 when dry)
     __shared__ double s_x[CLEAR ? 2 : 1][CLEAR || TOL ? CH : 1];
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
     const int lane = t & 63, wave = t >> 6;
     // the hypotenuse normals of plotter types 1..8 point to 90, 135, ... degrees
     if (t < 16) s_dir[t >> 1][t & 1] = c_normal[((((t >> 1) - 2) & 7) + 9) * 6 + 2 + (t & 1)];
-    for (int i = t; i < 64; i += CH) s_leg[i] = c_leg[i];
+    for (int i = t; i < 64; i += NT) s_leg[i] = c_leg[i];
 
     // XCD-aware order: virtual block v runs on XCD v % 8 (the dispatcher deals
     // workgroups round robin and the grid is a multiple of 8); XCD x owns a
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         if (!RAW && a.prev_max) {
             const int n = a.chunk_scen ? (int)sc.nchunks : a.prev_chunks;
             const double *const pm = a.prev_max + (a.chunk_scen ? sc.chunk_off : 0);
-            for (int i0 = t; i0 < n; i0 += CH) fastest = max_f64(fastest, pm[i0]);
+            for (int i0 = t; i0 < n; i0 += NT) fastest = max_f64(fastest, pm[i0]);
         }
 
         int32_t nb[3] = {-1, -1, -1};
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         // RAW: the chunk's neighbours, for the back edges; the flux slots are
         // not written before the edge loop
         int32_t *const s_nbr = reinterpret_cast<int32_t *>(&s_f[0][0][0]);
-        if (RAW) {
+        if (RAW && t < CH) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) s_nbr[k * CH + t] = nb[k];
         }
@@ -322,7 +324,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
 
         __builtin_amdgcn_s_setprio(0);
         // One pass over the list.  FIRST: a GeoClaw kernel's pass with clear_flux,
-        // which leaves the rounds (of CH entries) where one of a wave's edges
+        // which leaves the rounds (of NT entries) where one of a wave's edges
         // is not clear to a second pass with the general solver; returns their
         // bits, the same for the whole wave.  A pass of its own keeps the
         // general solver's registers from adding to the shortcut's.
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(4))) void eu
         constexpr bool FIRST = decltype(first_pass)::value;
         constexpr bool SHORT = GEOCLAW && FIRST;
         uint32_t rest = 0, bit = 1;
-        for (int e = t; e < total; e += CH, bit <<= 1) {
+        for (int e = t; e < total; e += NT, bit <<= 1) {
             if (!FIRST && !(rounds & bit)) continue;
             const uint32_t ent = s_list[e];
             const int lc = ent & 511, k = (ent >> 9) & 3, dir = (ent >> 22) & 7;
@@ -654,24 +656,38 @@ hipError_t launch_finalize(const StepArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <int SOLVER, int CH, int NT>
+static void launch_nt(const StepArgs &a, unsigned blocks, hipStream_t s) {
+    constexpr bool GEOCLAW = SOLVER == 0 || SOLVER == 1;  // the toleranced solvers
+    if (GEOCLAW && a.tol) {
+        if (a.flag_jumps)
+            hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, NT, true, false, GEOCLAW>),
+                               dim3(blocks), dim3(NT), 0, s, a);
+        else
+            hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, NT, false, false, GEOCLAW>),
+                               dim3(blocks), dim3(NT), 0, s, a);
+    } else if (a.flag_jumps)
+        hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, NT, true>), dim3(blocks), dim3(NT), 0, s,
+                           a);
+    else
+        hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, NT, false>), dim3(blocks), dim3(NT), 0,
+                           s, a);
+}
+
 template <int SOLVER, int CH>
 static void launch_t(const StepArgs &a, int64_t grid_blocks, hipStream_t s) {
     const int64_t nvirt = 8 * ((a.nchunks + 7) / 8);
     const int64_t blocks = grid_blocks > 0 && grid_blocks < nvirt ? grid_blocks : nvirt;
-    constexpr bool GEOCLAW = SOLVER == 0 || SOLVER == 1;  // the toleranced solvers
-    if (GEOCLAW && a.tol) {
-        if (a.flag_jumps)
-            hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, true, false, GEOCLAW>),
-                               dim3((unsigned)blocks), dim3(CH), 0, s, a);
-        else
-            hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, false, false, GEOCLAW>),
-                               dim3((unsigned)blocks), dim3(CH), 0, s, a);
-    } else if (a.flag_jumps)
-        hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, true>), dim3((unsigned)blocks), dim3(CH),
-                           0, s, a);
+    // Two threads per cell where every workgroup is resident at once that way
+    // (256 CUs of 1024 lanes at this kernel's registers): a chunk's ~1.6 CH
+    // edges then take one round instead of two, and the launch is as long as
+    // its slowest chunk.  100 steps: 1.38 -> 1.25 ms at 32 chunks, 1.54 ->
+    // 1.40 at 256, 1.79 -> 1.72 at 512; 2.42 -> 2.87 at 1024, and a full
+    // chip's step 134 -> 200 us.
+    if (CH <= 256 && a.nchunks * 2 * CH <= 256 * 1024)
+        launch_nt<SOLVER, CH, CH <= 256 ? 2 * CH : CH>(a, (unsigned)blocks, s);
     else
-        hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, false>), dim3((unsigned)blocks),
-                           dim3(CH), 0, s, a);
+        launch_nt<SOLVER, CH, CH>(a, (unsigned)blocks, s);
     if (!a.skip_finalize)
         hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)a.n_scen), dim3(FIN_THREADS), 0, s, a);
 }
@@ -691,7 +707,7 @@ template <int SOLVER>
 static void launch_raw_t(const StepArgs &a, hipStream_t s) {
     constexpr int CH = DEFAULT_CHUNK;
     const int64_t nvirt = 8 * ((a.nchunks + 7) / 8);
-    hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, false, true>), dim3((unsigned)nvirt),
+    hipLaunchKernelGGL((euler_step_kernel<SOLVER, CH, CH, false, true>), dim3((unsigned)nvirt),
                        dim3(CH), 0, s, a);
     hipLaunchKernelGGL(finalize_kernel, dim3(1), dim3(FIN_THREADS), 0, s, a);
 }

@@ -220,6 +220,7 @@ struct Batch {
     int pp = 0;
     int64_t pend_chunks = 0;
     int64_t part_cap = 0;
+    swe::Meet *d_meet = nullptr;      // [nscen * MEET_SLOTS], zero between launches
     double *eta[2] = {nullptr, nullptr}, *hu[2] = {nullptr, nullptr}, *hv[2] = {nullptr, nullptr};
     double *b = nullptr;
     int32_t *nbr = nullptr;
@@ -293,6 +294,7 @@ void release(Batch &B) {
     (void)hipFree(B.d_part_max[0]);
     (void)hipFree(B.d_part_max[1]);
     (void)hipFree(B.d_part_nref);
+    (void)hipFree(B.d_meet);
     (void)hipFree(B.b2);
     (void)hipFree(B.nbr2);
     (void)hipFree(B.plotter2);
@@ -467,7 +469,8 @@ int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
          hipMalloc(&B.refine, (size_t)B.ncells) == hipSuccess &&
          hipMalloc(&B.d_scen, sizeof(swe::Scen) * (size_t)nscen) == hipSuccess &&
          hipMalloc(&B.d_slots, sizeof(swe::Slots) * (size_t)nscen) == hipSuccess &&
-         hipMalloc(&B.d_dt, sizeof(double) * (size_t)nscen) == hipSuccess;
+         hipMalloc(&B.d_dt, sizeof(double) * (size_t)nscen) == hipSuccess &&
+         hipMalloc(&B.d_meet, sizeof(swe::Meet) * swe::MEET_SLOTS * (size_t)nscen) == hipSuccess;
     if (!ok) return fail(SWE_ERR_NOMEM, "device allocation of %lld cells failed", (long long)B.ncells);
     for (size_t i = 0; i < packs.size(); ++i) {
         const swe_mesh_desc &d = *topo_src[i];
@@ -481,6 +484,7 @@ int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
     std::vector<swe::Slots> init((size_t)nscen);
     HIP_TRY(hipMemcpy(B.d_slots, init.data(), sizeof(swe::Slots) * init.size(),
                       hipMemcpyHostToDevice));
+    HIP_TRY(hipMemset(B.d_meet, 0, sizeof(swe::Meet) * swe::MEET_SLOTS * (size_t)nscen));
     B.uploaded.assign((size_t)nscen, 0);
     B.cap = B.ncells;
     return rebuild_chunks(B);
@@ -546,6 +550,13 @@ int batch_download(Batch &B, int32_t s, double *eta, double *hu, double *hv, dou
     return SWE_OK;
 }
 
+// The meeting points of a step of few chunks per scenario, else null.
+swe::Meet *meet_of(const Batch &B) {
+    for (auto &s : B.scen)
+        if (s.nchunks > swe::MEET_CHUNKS) return nullptr;
+    return B.d_meet;
+}
+
 // One traversal with host-chosen dt per scenario; results per scenario.
 int batch_step(Batch &B, const double *dt, int forward, double *dt_cfl, int64_t *n_refine,
                int8_t *refine_host) {
@@ -555,6 +566,7 @@ int batch_step(Batch &B, const double *dt, int forward, double *dt_cfl, int64_t 
                            B.stream));
     swe::StepArgs a = make_args(B, B.cur, 1 - B.cur, forward);
     a.dt_host = B.d_dt;
+    a.meet = meet_of(B);
     a.refine = (refine_host || B.keep_flags) ? B.refine : nullptr;
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, B.stream));
     std::vector<swe::Slots> res((size_t)B.nscen);
@@ -622,6 +634,8 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
             a.part_max = B.d_part_max[1 - pp];
             a.prev_max = prev ? B.d_part_max[pp] : nullptr;
             a.prev_chunks = (int32_t)B.pend_chunks;
+        } else {
+            a.meet = meet_of(B);
         }
         return swe::launch_step(a, B.solver, B.chunk, B.grid, st);
     };
@@ -1004,6 +1018,7 @@ int batch_forward_device(Batch &B, const double *eta, const double *hu, const do
     a.masks = masks;
     a.out_dtcfl = dt_cfl_dev;
     a.skip_finalize = dt_cfl_dev ? 0 : 1;  // dt comes from the caller: no result is read
+    a.meet = dt_cfl_dev ? meet_of(B) : nullptr;
     a.tol = 0;  // the adjoint's sweeps: the rounding its kernels differentiate
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, st));
     return SWE_OK;
@@ -1314,6 +1329,7 @@ int swe_step_device(swe_handle *h, const double *eta, const double *hu, const do
     a.refine = refine_dev;
     a.out_dtcfl = dt_cfl_dev;
     a.out_nref = n_refine_dev;
+    a.meet = meet_of(B);
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, s));
     return SWE_OK;
 }

@@ -23,6 +23,27 @@ struct Slots {
     long long res_nref;          // refinement count of the last step
 };
 
+// Meeting point of a launch's workgroups that reduce a scenario's partials
+// themselves (StepArgs::meet): the largest partial's bits, and the workgroups
+// that came (low half) with their refinement counts (high half).  Both are 0
+// between launches: the last workgroup puts them back.
+struct alignas(128) Meet {
+    unsigned long long fastest, came;
+};
+// Per scenario: one that the results leave from, and MEET_FAN that workgroups
+// come to first where there are more of them (device-wide atomics on one
+// line take 30 ns each).
+constexpr int MEET_FAN = 16;
+constexpr int MEET_SLOTS = 1 + MEET_FAN;
+// Largest number of chunks per scenario that meet; above, a finalize kernel
+// reduces the partials.  Its launch costs 3.5 us on the host and as much
+// between the steps; a workgroup that meets holds its place 1-2 us longer.  A
+// step, us: 12.1 -> 10.7 at 128 chunks, 20.8 -> 17.3 at 1024, 45.8 -> 42.9 at
+// 4096, but 64.9 -> 66.5 at 8192 and 135 -> 139 at 16384 (32 or 64 places
+// instead of 16 change no figure by 1 %).  Steps on three streams at 328
+// chunks, bound by the host: 9.1 -> 5.4 us each.
+constexpr int64_t MEET_CHUNKS = 4096;
+
 // One scenario (mesh + constants) of a batch.  A single mesh is a batch of
 // one.  Scenarios of equal meshes share one copy of the topology.
 struct Scen {
@@ -70,6 +91,9 @@ struct StepArgs {
     int chained;
     int32_t prev_chunks;
     const double *prev_max;
+    // [n_scen * MEET_SLOTS]: the last workgroup of each scenario publishes
+    // the results; no finalize kernel follows.  Null: one does.
+    Meet *meet;
     // refinement flags from surface-elevation jumps between wet neighbours
     // of the state the step reads (refine above jump_refine, coarsen below
     // jump_coarsen) instead of volume_op's |dQ_h| criterion
@@ -205,8 +229,8 @@ hipError_t launch_finalize(const StepArgs &a, hipStream_t s);
 // the partials of the step before.  Every workgroup reads all of them, so a
 // chain trades the finalize kernel (4-5 us with its launch) for nchunks^2
 // reads from L2.  100 steps: 1.33 -> 1.06 ms at 128 chunks, 2.81 -> 2.39 at
-// 1024, 4.24 -> 4.11 at 2048, but 6.75 -> 7.56 at 4096.
-constexpr int64_t CHAIN_CHUNKS = 2048;
+// 1024; at 2048, 4.24 -> 4.15, and 4.05 where the workgroups meet instead.
+constexpr int64_t CHAIN_CHUNKS = 1024;
 // The step of a single mesh whose nbr holds plain neighbour cells
 // (StepArgs::raw_nbr), chunk DEFAULT_CHUNK, one workgroup per chunk, flags
 // by volume_op's criterion; then the finalize kernel.

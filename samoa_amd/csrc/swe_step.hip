@@ -96,6 +96,39 @@ __device__ __forceinline__ double next_dt(double courant, double dt_clamp, doubl
     return dt_clamp > 0.0 ? dmin2(dt_clamp, next) : next;
 }
 
+// One workgroup's partials meet the others' (cl: its chunk among the n of the
+// scenario).  Returns true in the last one, with the scenario's values.
+// Relaxed device-wide atomics in program order: each returns before the next
+// is issued (the empty asm needs its result).
+__device__ __forceinline__ bool meet(Meet *f, uint32_t cl, uint32_t n, double &fastest,
+                                     long long &refined) {
+    auto bits = (unsigned long long)__double_as_longlong(fastest);
+    unsigned long long inc = 1ull | ((unsigned long long)refined << 32);
+    auto come = [&](Meet *m, uint32_t expected) -> bool {
+        const unsigned long long seen = __hip_atomic_fetch_max(&m->fastest, bits, __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::"v"(seen) : "memory");
+        const unsigned long long old =
+            __hip_atomic_fetch_add(&m->came, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)old + 1u != expected) return false;
+        asm volatile("" ::: "memory");
+        bits = __hip_atomic_exchange(&m->fastest, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&m->came, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        inc = 1ull | (((old >> 32) + (inc >> 32)) << 32);
+        return true;
+    };
+    if (n > MEET_FAN) {
+        const uint32_t k = cl % MEET_FAN;
+        if (!come(f + 1 + k, (n - k + MEET_FAN - 1) / MEET_FAN)) return false;
+        if (!come(f, MEET_FAN)) return false;
+    } else if (!come(f, n)) {
+        return false;
+    }
+    fastest = __longlong_as_double((long long)bits);
+    refined = (long long)(inc >> 32);
+    return true;
+}
+
 // Lanes of the mask below this one.
 __device__ __forceinline__ int lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
@@ -566,8 +599,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 m = max_f64(m, s_wmax[w]);
                 rsum += s_wref[w];
             }
-            a.part_max[chunk] = m;
-            a.part_nref[chunk] = rsum;
+            if (!RAW && a.meet) {
+                long long all = rsum;
+                if (meet(a.meet + (int64_t)s * MEET_SLOTS, chunk - (uint32_t)sc.chunk_off,
+                         (uint32_t)sc.nchunks, m, all)) {
+                    const double c = cfl_minimum(sc.scaling, m);
+                    a.slots[s].res_dtcfl = c;
+                    a.slots[s].res_nref = all;
+                    if (a.out_dtcfl) a.out_dtcfl[s] = c;
+                    if (a.out_nref) a.out_nref[s] = all;
+                    if (a.device_dt) {
+                        a.slots[s].time = a.slots[s].time + dt;
+                        a.slots[s].dt = next_dt(sc.courant, sc.dt_clamp, c);
+                    }
+                }
+            } else {
+                a.part_max[chunk] = m;
+                a.part_nref[chunk] = rsum;
+            }
         }
         __syncthreads();  // LDS is reused by the next chunk
     }
@@ -688,7 +737,7 @@ static void launch_t(const StepArgs &a, int64_t grid_blocks, hipStream_t s) {
         launch_nt<SOLVER, CH, CH <= 256 ? 2 * CH : CH>(a, (unsigned)blocks, s);
     else
         launch_nt<SOLVER, CH, CH>(a, (unsigned)blocks, s);
-    if (!a.skip_finalize)
+    if (!a.skip_finalize && !a.meet)
         hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)a.n_scen), dim3(FIN_THREADS), 0, s, a);
 }
 

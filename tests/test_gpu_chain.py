@@ -48,10 +48,11 @@ class HostChain:
             self.fwd = not self.fwd
 
 
-# one chunk, ragged, few chunks; the largest chain (2048 chunks of 256 cells)
-# and, with 128-cell chunks, the smallest mesh without one
+# one chunk, ragged, few chunks; the largest chain (1024 chunks of 256 cells);
+# the smallest (2048) and largest (4096) meshes whose workgroups meet, and,
+# with 128-cell chunks, one with a finalize kernel (8192)
 @pytest.mark.parametrize("depth,chunk", [(0, None), (5, None), (7, 128), (10, 512), (12, None),
-                                         (18, None), (18, 128)])
+                                         (17, None), (18, None), (18, 128), (19, 128)])
 @pytest.mark.parametrize("parts", [[5], [1, 4], [2, 3], [1, 1, 1, 1, 1]])
 def test_pieces_of_a_run_equal_single_traversals(depth, chunk, parts):
     print("case:", depth, chunk, parts, flush=True)
@@ -122,7 +123,7 @@ def test_other_calls_between_the_pieces():
 def test_remeshing_between_the_pieces():
     """The step after a remeshing forms its dt from the old mesh's partials,
     also where the new mesh needs more room or leaves the chain's range."""
-    for depth, dmax in ((6, 9), (17, 19)):
+    for depth, dmax in ((6, 9), (16, 18), (18, 20)):
         print("case:", depth, flush=True)
         mesh = host.mesh_uniform(depth)
         st = beach(mesh, 2)
@@ -170,6 +171,35 @@ def test_batch_of_uneven_meshes():
             assert np.array_equal(x, y)
         r.op.close()
     b.close()
+
+
+# cells per chunk x chunks around the number of places workgroups meet at
+@pytest.mark.parametrize("grid", [0, 8])
+@pytest.mark.parametrize("depth,chunk", [(3, 128), (11, 256), (11, 128), (12, 512), (14, 256),
+                                         (19, 256), (19, 128)])
+def test_single_steps_publish_their_results(depth, chunk, grid):
+    """dt_cfl and the refinement count of repeated steps do not depend on how
+    the workgroups' partials are reduced: equal to the counted flags and to
+    the other launch shapes', with the places left clean for the next step."""
+    print("case:", depth, chunk, grid, flush=True)
+    meshes = [host.mesh_uniform(depth)]
+    op = swe.EulerTimestep(meshes[0], scaling=1e3, dry_tolerance=1e-3, min_depth=depth - 1,
+                           max_depth=depth + 6, boundary=swe.BC_WALL)
+    st = beach(meshes[0], 5)
+    dt = 0.4 * host.initial_dt(meshes[0], st, COURANT) * 1e3
+    got = []
+    for c, g in ((chunk, grid), (256, 0), (512, 16)):
+        op.set_tuning(c, g)
+        op.upload(*st)
+        rows = []
+        for k in range(3):
+            res = op.traverse(dt, k % 2 == 0, flags=True)
+            assert res.n_refine == int((res.refine == 1).sum())
+            rows.append((res.dt_cfl, res.n_refine))
+        got.append(rows)
+    assert got[0] == got[1] == got[2]
+    assert depth < 8 or got[0][0][1] > 0
+    op.close()
 
 
 def test_cells_without_numbers_set_no_limit():

@@ -216,7 +216,7 @@ class GaugeInversion:
         # Two-level checkpointing, pipelined: the recompute of segment j - 1
         # runs on a side stream while the adjoint sweeps segment j on the
         # current stream, in the other of two segment buffers.  The two
-        # kernels then share the GPU (the adjoint kernel alone holds two
+        # kernels then share the GPU (the adjoint kernel alone holds three
         # waves per SIMD).  Events order every buffer's reuse.
         checkpoints = tape["checkpoints"]
         starts = sorted(checkpoints)

@@ -18,10 +18,25 @@
 // per-(cell, edge) LDS slots, summed per cell in a fixed order (so results do
 // not depend on scheduling).  Edges to cells of other chunks are solved by
 // both chunks, each keeping its own side.
+//
+// What bounds it: FP64 vector issue.  Most edges are clearly subcritical: they
+// take clear_flux_adj (660 vector instructions with staging and scatter, the
+// same results), the others are compacted into a second list for
+// edge_flux_adj (about 1700).  On the d20 tsunami (2.1 M cells) this took the
+// kernel from 2740 to 1250 vector instructions per 64 cells, a beach's (d18, a
+// fifth of it dry) from 61 to 35 us.  The general pass alone needs 206
+// registers: held to 168 it spills 76 bytes on its few edges, and three waves
+// per SIMD instead of two hide more of the first pass's LDS and memory waits:
+// 213.7 us at the start, 122 with two waves, 106 with three.  LDS (50 KB for
+// 256 cells) allows no fourth.  The f-wave kernel went from 107 to 81 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "swe_adjoint.hpp"
+#include "swe_adjoint_clear.hpp"
+#include "swe_device.hpp"
 #include "swe_internal.hpp"
 
 namespace swe {
@@ -30,231 +45,305 @@ namespace swe {
 __constant__ double c_normal_adj[17 * 3 * 2];  // [plotter + 8][edge][x,y]
 __constant__ double c_leg_adj[64];             // l(k) = sqrt(0.5)**k at k + 1
 
+// (the LDS of 512 cells allows two waves per SIMD)
 template <int SOLVER, int CH>
-__global__ __launch_bounds__(CH) void adjoint_step_kernel(AdjArgs a) {
-    __shared__ double s_q[4][CH];        // eta, hu, hv, b of the chunk at t_n
-    __shared__ double s_seed[3][CH];     // s * lam^{n+1} after the limiter (per cell)
-    __shared__ double s_gb[SOLVER != 1 ? CH : 1];  // each cell's b gradient so far
-    __shared__ double s_g[4][3][CH];     // transpose-flux contributions per (edge, cell)
-    __shared__ int32_t s_nbr[3][CH];
-    __shared__ int8_t s_plot[CH];
-    __shared__ int8_t s_dep[CH];
-    __shared__ uint16_t s_list[3 * CH];
-    __shared__ int s_wsum[CH / 64];
-
-    __shared__ double s_normal[17 * 3 * 2];  // geometry tables in LDS (see swe_step.hip)
+__global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(CH == 512 ? 2 : 3))) void
+adjoint_step_kernel(AdjArgs args) {
+    __shared__ double s_q[4][CH];     // eta, hu, hv, b of the chunk at t_n
+    __shared__ double s_x[2][CH];     // 1/h and sqrt(g h) of each cell (clear_cell)
+    __shared__ double s_seed[3][CH];  // s * lam^{n+1} after the limiter (per cell)
+    __shared__ double s_gb[CH];       // each cell's b gradient so far
+    __shared__ double s_g[4][3][CH];  // transpose-flux contributions per (edge, cell)
+    // The edges to solve, as in the step kernel: those inside the chunk, then
+    // those leaving it, then the packed neighbours of the latter.
+    __shared__ uint32_t s_list[3 * CH + 4];
+    __shared__ uint16_t s_rest[3 * CH];  // entries left to the general solver
+    __shared__ int8_t s_dep[CH], s_mask[CH];
+    __shared__ int s_wsum[CH / 64], s_nrest;
+    __shared__ double s_dir[8][2];  // the unit vectors at multiples of 45 degrees
     __shared__ double s_leg[64];
 
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const double g = a.g, inv16g = a.inv16g;
-    for (int i = t; i < 17 * 3 * 2; i += CH) s_normal[i] = c_normal_adj[i];
+    int t = threadIdx.x;
+    if (t < 16) s_dir[t >> 1][t & 1] = c_normal_adj[((((t >> 1) - 2) & 7) + 9) * 6 + 2 + (t & 1)];
     for (int i = t; i < 64; i += CH) s_leg[i] = c_leg_adj[i];
-    __syncthreads();
-    const int64_t nchunks = a.nchunks;
-    const int64_t q = nchunks / 8, r = nchunks % 8;
-    const int64_t nvirt = 8 * ((nchunks + 7) / 8);
-    for (int64_t v = blockIdx.x; v < nvirt; v += gridDim.x) {
-        const int64_t xcd = v % 8, i = v / 8;
+    const uint32_t nchunks = (uint32_t)args.nchunks, q = nchunks / 8, r = nchunks % 8;
+    const uint32_t nvirt = 8 * ((nchunks + 7) / 8);
+    for (uint32_t v = blockIdx.x; v < nvirt; v += gridDim.x) {
+        const uint32_t xcd = v % 8, i = v / 8;
         if (i >= q + (xcd < r ? 1 : 0)) continue;
-        const int64_t chunk = xcd * q + (xcd < r ? xcd : r) + i;
+        const uint32_t chunk = xcd * q + (xcd < r ? xcd : r) + i;
+        // read where they are used, for each chunk (see the step kernel)
+        auto ap = (const __attribute__((address_space(4))) AdjArgs *)
+            __builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(ap));
+        const auto &a = *ap;
+        // and what follows from t is computed where it is used: LDS addresses
+        // kept across the loops are registers that the general solver lacks
+        asm volatile("" : "+v"(t));
+        const int lane = t & 63, wave = t >> 6;
         // raised wave priority for the chunk's loads and edge list, as in the
         // forward step kernel
         __builtin_amdgcn_s_setprio(2);
-        const int s = a.chunk_scen ? a.chunk_scen[chunk] : 0;
-        const Scen sc = a.scen[s];
-        const int64_t lbase = (chunk - sc.chunk_off) * CH;
+        const int s = a.chunk_scen ? scalar(a.chunk_scen)[chunk] : 0;
+        const auto &sc = *(scalar(a.scen) + s);
+        const int32_t lbase = (int32_t)(chunk - (uint32_t)sc.chunk_off) * CH;
         const int cnt = (int)((sc.n - lbase) < CH ? (sc.n - lbase) : CH);
         const bool active = t < cnt;
-        const int64_t lc_t = lbase + t;
         const int64_t gs = sc.cell_off, gt = sc.topo_off;
-        const double dt = a.dt_dev ? a.dt_dev[s] : a.dt;
-        const double drytol = sc.drytol, S = sc.scaling;
+        const double g = a.g, drytol = sc.drytol, S = sc.scaling;
+        const double dt = a.dt_dev ? scalar(a.dt_dev)[s] : a.dt;
 
         // transpose of the cell update for this thread's cell
         int32_t nb[3] = {-1, -1, -1};
-        int8_t plot = 1, dep = 0;
-        double dir_e = 0.0, dir_u = 0.0, dir_v = 0.0, dir_b = 0.0;
+        int plot = 1;
         if (active) {
             // every load in one round: the state, topology, masks and
             // adjoint inputs first, the depth (behind a branch) last
-            const int64_t x = gs + lc_t;
+            const int64_t x = gs + lbase + t;
             const double qe = a.eta[x], qu = a.hu[x], qv = a.hv[x], qb = a.b[x];
             const int mk = a.masks[x];
             const double le = a.leta[x], lu = a.lhu[x], lv = a.lhv[x];
             // only this cell's thread adds to its b gradient: read now, with
-            // the other loads, not after the edge loop (the f-wave kernel, at
-            // 168 VGPRs and three waves per SIMD, reads it at the end: the
-            // staged read costs it a register and a wave)
-            if constexpr (SOLVER != 1) s_gb[t] = a.gb[x];
-            nb[0] = a.nbr[3 * (gt + lc_t)];
-            nb[1] = a.nbr[3 * (gt + lc_t) + 1];
-            nb[2] = a.nbr[3 * (gt + lc_t) + 2];
-            plot = a.plotter[gt + lc_t];
-            dep = (int8_t)(sc.depth >= 0 ? sc.depth : a.depth[gt + lc_t]);
+            // the other loads, not after the edge loop
+            s_gb[t] = a.gb[x];
+            const int32_t *const nbr = a.nbr + 3 * (gt + lbase);
+            nb[0] = nbr[3 * t];
+            nb[1] = nbr[3 * t + 1];
+            nb[2] = nbr[3 * t + 2];
+            plot = a.plotter[gt + lbase + t];
+            const int dep = sc.depth >= 0 ? sc.depth : (int)a.depth[gt + lbase + t];
+            s_dep[t] = (int8_t)dep;
             s_q[0][t] = qe;
             s_q[1][t] = qu;
             s_q[2][t] = qv;
             s_q[3][t] = qb;
-            double g2e = le, g2u = lu, g2v = lv;
-            if (mk & 2) {  // drying fix: eta = min(b, 0), p = 0
-                g2e = g2u = g2v = 0.0;
-                if (qb < 0.0) dir_b += le;
-            }
-            if (mk & 1) {  // wetting fix: eta = b + drytol, p = 0 before the update
-                dir_b += g2e;
-            } else {
-                dir_e = g2e;
-                dir_u = g2u;
-                dir_v = g2v;
-            }
+            const ClearCell cc = clear_cell(qe, qu, qv, qb, drytol, g);
+            s_x[0][t] = cc.r;
+            s_x[1][t] = cc.c;
+            s_mask[t] = (int8_t)mk;
+            const bool dry = (mk & 2) != 0;  // drying fix: eta = min(b, 0), p = 0
             const double vol = (S * S) * ldexp(1.0, -(dep + 1));
             const double scale = -dt / vol;
-            s_seed[0][t] = scale * g2e;
-            s_seed[1][t] = scale * g2u;
-            s_seed[2][t] = scale * g2v;
+            s_seed[0][t] = scale * (dry ? 0.0 : le);
+            s_seed[1][t] = scale * (dry ? 0.0 : lu);
+            s_seed[2][t] = scale * (dry ? 0.0 : lv);
         }
-        s_nbr[0][t] = nb[0];
-        s_nbr[1][t] = nb[1];
-        s_nbr[2][t] = nb[2];
-        s_plot[t] = plot;
-        s_dep[t] = dep;
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int m = 0; m < 4; ++m) s_g[m][k][t] = 0.0;
+        if (t == 0) s_nrest = 0;
 
-        int own = 0;
+        // Edges this thread's cell must solve: those leaving the chunk, and
+        // the inner ones whose other cell the traversal visits later (so from
+        // their left side).
+        int inner = 0, leave = 0;
         if (active) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const int32_t p = nb[k];
-                const int64_t o = (int64_t)(p >> 2);
-                const bool inside = p >= 0 && o >= lbase && o < lbase + cnt;
-                if (!inside || o > lc_t) own |= 1 << k;
+                const int lo = (p >> 2) - lbase;  // chunk-local neighbour
+                if (!(p >= 0 && (uint32_t)lo < (uint32_t)cnt)) leave |= 1 << k;
+                else if (a.forward ? lo > t : lo < t) inner |= 1 << k;
             }
         }
-        const int nown = __popc(own);
-        const uint64_t b0 = __ballot(nown & 1), b1 = __ballot(nown & 2);
-        const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-        const int wpre = __popcll(b0 & lt) + 2 * __popcll(b1 & lt);
-        if (lane == 0) s_wsum[wave] = __popcll(b0) + 2 * __popcll(b1);
+        // workgroup exclusive prefixes of both counts (0..3 each) via ballots,
+        // packed: inner in the low half, leaving in the high half
+        const int nin = __popc(inner), nout = __popc(leave);
+        const uint64_t i0 = __ballot(nin & 1), i1 = __ballot(nin & 2);
+        const uint64_t o0 = __ballot(nout & 1), o1 = __ballot(nout & 2);
+        const int wpre = lanes_below(i0) + 2 * lanes_below(i1) +
+                         ((lanes_below(o0) + 2 * lanes_below(o1)) << 16);
+        if (lane == 0)
+            s_wsum[wave] = __popcll(i0) + 2 * __popcll(i1) +
+                           ((__popcll(o0) + 2 * __popcll(o1)) << 16);
         __syncthreads();
-        int pre = wpre, total = 0;
+        int pre = wpre, sum = 0;
 #pragma unroll
         for (int w = 0; w < CH / 64; ++w) {
             const int ws = s_wsum[w];
             pre += w < wave ? ws : 0;
-            total += ws;
+            sum += ws;
         }
+        const int n_inner = sum & 0xffff, total = n_inner + (sum >> 16);
+        int pi = pre & 0xffff, po = n_inner + (pre >> 16);
+        const int turn = plot < 0 ? -plot : plot;  // edge normals: see the step kernel
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (own & (1 << k)) s_list[pre++] = (uint16_t)((t << 2) | k);
+        for (int k = 0; k < 3; ++k) {
+            const int d0 = k == 1 ? 1 : ((k == 0) == (plot > 0) ? 4 : 6);
+            const int32_t p = nb[k];
+            const bool in = inner & (1 << k), out = leave & (1 << k);
+            const uint32_t other =
+                in ? ((uint32_t)((p >> 2) - lbase) << 11) | ((uint32_t)(p & 3) << 20)
+                   : LEAVES | (p < 0 ? BOUNDARY : 0u);
+            if (in || out)
+                s_list[in ? pi : po] = (uint32_t)t | ((uint32_t)k << 9) |
+                                       ((uint32_t)((turn + d0) & 7) << 22) | other;
+            if (out) s_list[po + total - n_inner] = (uint32_t)p;
+            pi += in ? 1 : 0;
+            po += out ? 1 : 0;
+        }
         __syncthreads();
 
         __builtin_amdgcn_s_setprio(0);
-        for (int e = t; e < total; e += CH) {
-            const int ent = s_list[e];
-            const int lc = ent >> 2, k = ent & 3;
-            const int64_t cc = lbase + lc;
-            const int32_t p = s_nbr[k][lc];
-            const int pi = s_plot[lc] + 8;
-            const double nx = s_normal[(pi * 3 + k) * 2], ny = s_normal[(pi * 3 + k) * 2 + 1];
-            const double qe = s_q[0][lc], qu = s_q[1][lc], qv = s_q[2][lc], qb = s_q[3][lc];
+        // One pass over the list (FIRST, clear_flux_adj; it lists the edges
+        // that are not clear) or over the rest (edge_flux_adj).  An edge's
+        // pass depends on its two states alone and each writes its own
+        // slots, so results depend neither on the chunking nor on the order
+        // of the rest.  Two passes: the general solver's registers do not
+        // add to the shortcut's.
+        auto solve = [&](auto first_pass, int n) {
+        constexpr bool FIRST = decltype(first_pass)::value;
+        asm volatile("" : "+v"(t), "+s"(ap));
+        const auto &a = *ap;
+        const double g = a.g;
+        for (int i = t; i < n; i += CH) {
+            const int e = FIRST ? i : s_rest[i];
+            const uint32_t ent = s_list[e];
+            const int lc = ent & 511, k = (ent >> 9) & 3, dir = (ent >> 22) & 7;
+            double nx = s_dir[dir][0], ny = s_dir[dir][1];
+            // both cells' state, 1/h and c, and seeds: left and right for an
+            // inner edge; one that leaves the chunk may need them exchanged
+            double L[6] = {}, R[6] = {}, fL[3], fR[3] = {0.0, 0.0, 0.0};
             const int dc = s_dep[lc];
-            const double len_c = S * (k == 1 ? s_leg[dc] : s_leg[dc + 1]);
-            const double sc0 = s_seed[0][lc] * len_c, sc1 = s_seed[1][lc] * len_c,
-                         sc2 = s_seed[2][lc] * len_c;
-            const bool bnd = p < 0;
-            const int64_t o = bnd ? cc : (int64_t)(p >> 2);
-            const int ko = p & 3;
-            const bool inside = !bnd && o >= lbase && o < lbase + cnt;
-            double oe, ou, ov, ob, so0 = 0.0, so1 = 0.0, so2 = 0.0;
-            if (bnd) {
-                oe = qe;
-                ob = qb;
-                ou = qu;
-                ov = qv;
-                if (a.bc == 1) {
-                    const double dp = qu * nx + qv * ny;
-                    ou = qu - (2.0 * dp) * nx;
-                    ov = qv - (2.0 * dp) * ny;
+            const double len = S * s_leg[k == 1 ? dc : dc + 1];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) L[m] = s_q[m][lc];
+            if (FIRST) {
+                L[4] = s_x[0][lc];
+                L[5] = s_x[1][lc];
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) fL[m] = s_seed[m][lc] * len;
+            const bool inside = !(ent & LEAVES);
+            const int lo = (ent >> 11) & 511, ko = (ent >> 20) & 3;
+            bool flip = false;
+            if (inside) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) R[m] = s_q[m][lo];
+                if (FIRST) {
+                    R[4] = s_x[0][lo];
+                    R[5] = s_x[1][lo];
                 }
-            } else if (inside) {
-                const int lo = (int)(o - lbase);
-                oe = s_q[0][lo];
-                ou = s_q[1][lo];
-                ov = s_q[2][lo];
-                ob = s_q[3][lo];
                 const int dl = s_dep[lo];
-                const double len_o = S * (ko == 1 ? s_leg[dl] : s_leg[dl + 1]);
-                so0 = s_seed[0][lo] * len_o;
-                so1 = s_seed[1][lo] * len_o;
-                so2 = s_seed[2][lo] * len_o;
+                const double len_o = S * s_leg[ko == 1 ? dl : dl + 1];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) fR[m] = s_seed[m][lo] * len_o;
+            } else if (ent & BOUNDARY) {
+#pragma unroll
+                for (int m = 0; m < 6; ++m) R[m] = L[m];
+                if (a.bc == 1) {
+                    const double dp = L[1] * nx + L[2] * ny;
+                    R[1] = L[1] - (2.0 * dp) * nx;
+                    R[2] = L[2] - (2.0 * dp) * ny;
+                }
             } else {
+                const int32_t p = (int32_t)s_list[e + total - n_inner], o = p >> 2;
                 const int64_t x = gs + o;
-                oe = a.eta[x];
-                ou = a.hu[x];
-                ov = a.hv[x];
-                ob = a.b[x];
+                R[0] = a.eta[x];
+                R[1] = a.hu[x];
+                R[2] = a.hv[x];
+                R[3] = a.b[x];
                 const int mk = a.masks[x];
                 // read with the rest, then selected (a read under the mask
                 // test would wait for the mask first)
                 const double l0 = a.leta[x], l1 = a.lhu[x], l2 = a.lhv[x];
                 const int dl = sc.depth >= 0 ? sc.depth : a.depth[gt + o];
+                if (FIRST) {
+                    const ClearCell y = clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+                    R[4] = y.r;
+                    R[5] = y.c;
+                }
                 // the neighbour's seed exactly as its own chunk forms it
                 // ((s * lam) after the limiter, times the edge length), so
                 // that results do not depend on the chunking
                 const double vol = (S * S) * ldexp(1.0, -(dl + 1));
                 const double scale = -dt / vol;
-                const double len_o = S * (ko == 1 ? s_leg[dl] : s_leg[dl + 1]);
+                const double len_o = S * s_leg[(p & 3) == 1 ? dl : dl + 1];
                 const bool dry = (mk & 2) != 0;
-                so0 = (scale * (dry ? 0.0 : l0)) * len_o;
-                so1 = (scale * (dry ? 0.0 : l1)) * len_o;
-                so2 = (scale * (dry ? 0.0 : l2)) * len_o;
+                fR[0] = (scale * (dry ? 0.0 : l0)) * len_o;
+                fR[1] = (scale * (dry ? 0.0 : l1)) * len_o;
+                fR[2] = (scale * (dry ? 0.0 : l2)) * len_o;
+                flip = a.forward ? o < lbase : o > lbase;  // the other cell comes first
             }
-            const bool c_left = bnd || (a.forward ? (cc < o) : (cc > o));
-            const double sx = c_left ? nx : -nx, sy = c_left ? ny : -ny;
-            // seeds of the left and right sides, selected element-wise (a
-            // pointer selection between two arrays would put them in scratch)
-            const double gfl[3] = {c_left ? sc0 : so0, c_left ? sc1 : so1, c_left ? sc2 : so2};
-            const double gfr[3] = {c_left ? so0 : sc0, c_left ? so1 : sc1, c_left ? so2 : sc2};
-            double gQL[4] = {0, 0, 0, 0}, gQR[4] = {0, 0, 0, 0};
-            edge_flux_adj<SOLVER>(sx, sy, c_left ? qe : oe, c_left ? qu : ou, c_left ? qv : ov,
-                                  c_left ? qb : ob, c_left ? oe : qe, c_left ? ou : qu,
-                                  c_left ? ov : qv, c_left ? ob : qb, drytol, g, inv16g,
-                                  gfl, gfr, gQL, gQR);
-            double gc[4], go[4];
+            const bool flips = __ballot(flip) != 0;  // no wave of inner edges does
+            if (flips) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                gc[m] = c_left ? gQL[m] : gQR[m];
-                go[m] = c_left ? gQR[m] : gQL[m];
+                for (int m = 0; m < 6; ++m) {
+                    const double x = L[m];
+                    L[m] = flip ? R[m] : x;
+                    R[m] = flip ? x : R[m];
+                }
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                    const double x = fL[m];
+                    fL[m] = flip ? fR[m] : x;
+                    fR[m] = flip ? x : fR[m];
+                }
+                nx = flip ? -nx : nx;
+                ny = flip ? -ny : ny;
             }
-            if (bnd) {  // the ghost is a function of this cell's state
-                gc[0] += go[0];
-                gc[3] += go[3];
+            double gL[4] = {0.0, 0.0, 0.0, 0.0}, gR[4] = {0.0, 0.0, 0.0, 0.0};
+            if constexpr (FIRST) {
+                const double hL = L[0] - L[3], hR = R[0] - R[3];
+                const ClearEdge ce = clear_edge(nx, ny, hL, L[1], L[2], L[4], hR, R[1], R[2], R[4]);
+                if (is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5])) {
+                    if (!clear_flux_adj<SOLVER>(nx, ny, ce, hL, L[3], L[4], L[5], hR, R[3], R[4],
+                                                R[5], g, fL, fR, gL, gR)) {
+                        s_rest[atomicAdd(&s_nrest, 1)] = (uint16_t)e;
+                        continue;
+                    }
+                } else if (!(hL <= drytol && hR <= drytol)) {
+                    s_rest[atomicAdd(&s_nrest, 1)] = (uint16_t)e;
+                    continue;
+                }
+            } else {
+                edge_flux_adj<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], R[0], R[1], R[2], R[3], drytol,
+                                      g, a.inv16g, fL, fR, gL, gR);
+            }
+            if (flips) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) gL[m] = flip ? gR[m] : gL[m];
+            }
+            if (ent & BOUNDARY) {  // the ghost is a function of this cell's state
+                gL[0] += gR[0];
+                gL[3] += gR[3];
                 if (a.bc == 1) {
-                    const double gdp = -2.0 * (go[1] * nx + go[2] * ny);
-                    gc[1] += go[1] + gdp * nx;
-                    gc[2] += go[2] + gdp * ny;
+                    const double gdp = -2.0 * (gR[1] * nx + gR[2] * ny);
+                    gL[1] += gR[1] + gdp * nx;
+                    gL[2] += gR[2] + gdp * ny;
                 } else {
-                    gc[1] += go[1];
-                    gc[2] += go[2];
+                    gL[1] += gR[1];
+                    gL[2] += gR[2];
                 }
             }
 #pragma unroll
-            for (int m = 0; m < 4; ++m) s_g[m][k][lc] = gc[m];
+            for (int m = 0; m < 4; ++m) s_g[m][k][lc] = gL[m];
             if (inside) {
-                const int lo = (int)(o - lbase);
 #pragma unroll
-                for (int m = 0; m < 4; ++m) s_g[m][ko][lo] = go[m];
+                for (int m = 0; m < 4; ++m) s_g[m][ko][lo] = gR[m];
             }
         }
+        };
+        solve(std::true_type{}, total);
         __syncthreads();
+        const int nrest = s_nrest;
+        if (nrest) {
+            solve(std::false_type{}, nrest);
+            __syncthreads();
+        }
 
-        if (active) {
-            const int64_t x = gs + lc_t;
-            double le = dir_e, lu = dir_u, lv = dir_v, lb = dir_b;
+        asm volatile("" : "+v"(t));
+        if (t < cnt) {
+            const int64_t x = gs + lbase + t;
+            // the limiter's own part, from a second read of the adjoint (in
+            // registers across the edge loop it costs a wave per SIMD)
+            const int mk = s_mask[t];
+            double le = a.leta[x], lu = a.lhu[x], lv = a.lhv[x], lb = 0.0;
+            if (mk & 2) {  // drying fix: eta = min(b, 0), p = 0
+                if (s_q[3][t] < 0.0) lb += le;
+                le = lu = lv = 0.0;
+            }
+            if (mk & 1) {  // wetting fix: eta = b + drytol, p = 0 before the update
+                lb += le;
+                le = lu = lv = 0.0;
+            }
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 le += s_g[0][k][t];
@@ -265,8 +354,7 @@ __global__ __launch_bounds__(CH) void adjoint_step_kernel(AdjArgs a) {
             a.leta_out[x] = le;
             a.lhu_out[x] = lu;
             a.lhv_out[x] = lv;
-            if constexpr (SOLVER != 1) a.gb[x] = s_gb[t] + lb;
-            else a.gb[x] += lb;
+            a.gb[x] = s_gb[t] + lb;
         }
         __syncthreads();  // LDS is reused by the next chunk
     }

@@ -91,7 +91,7 @@ struct ClearCell {
 
 // Gravitational constants the shortcuts are derived for (the whole launch
 // takes the general path otherwise).
-constexpr double CLEAR_MIN_G = 1.0e-3, CLEAR_MAX_G = 1.0e3;
+constexpr double CLEAR_MIN_G = 0x1p-10, CLEAR_MAX_G = 0x1p10;
 
 SWE_HD ClearCell clear_cell(double eta, double hu, double hv, double b, double drytol, double g) {
     const double h = eta - b;
@@ -106,16 +106,19 @@ SWE_HD ClearCell clear_cell(double eta, double hu, double hv, double b, double d
 #if defined(__HIP_DEVICE_COMPILE__)
     e = __builtin_amdgcn_frexp_exp(hu);
     const int e1 = __builtin_amdgcn_frexp_exp(hv), e2 = __builtin_amdgcn_frexp_exp(b);
+    // CLEAR_MIN_G <= g < CLEAR_MAX_G by the high words: scalar instructions
+    const bool g_fits = (uint32_t)__double2hiint(g) - (uint32_t)__double2hiint(CLEAR_MIN_G) <
+                        (uint32_t)__double2hiint(CLEAR_MAX_G) - (uint32_t)__double2hiint(CLEAR_MIN_G);
 #else
     int e1, e2;
     (void)frexp(hu, &e);
     (void)frexp(hv, &e1);
     (void)frexp(b, &e2);
+    const bool g_fits = g >= CLEAR_MIN_G && g < CLEAR_MAX_G;
 #endif
     e = e < e1 ? e : e1;
     e = e < e2 ? e : e2;
-    const bool tame = e > -240 && fabs(hu) + fabs(hv) + fabs(b) < 0x1p60 && h < 0x1p40 &&
-                      g >= CLEAR_MIN_G && g <= CLEAR_MAX_G;
+    const bool tame = e > -240 && fabs(hu) + fabs(hv) + fabs(b) < 0x1p60 && h < 0x1p40 && g_fits;
     if (!tame) k.c = __builtin_nan("");
     return k;
 }

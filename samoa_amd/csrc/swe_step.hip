@@ -42,6 +42,7 @@
 
 #include <type_traits>
 
+#include "swe_device.hpp"
 #include "swe_internal.hpp"
 #include "swe_riemann.hpp"
 #include "swe_riemann_clear.hpp"
@@ -51,13 +52,6 @@ namespace swe {
 
 __constant__ double c_normal[17 * 3 * 2];  // [plotter + 8][edge][x,y]
 __constant__ double c_leg[64];             // l(k) = sqrt(0.5)**k at k + 1
-
-// A pointer to memory that no kernel writes while this one runs, for scalar
-// loads from uniform addresses.
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T *scalar(const T *p) {
-    return (const __attribute__((address_space(4))) T *)p;
-}
 
 // v_max_f64 without the quieting of signalling NaN that fmax adds.
 __device__ __forceinline__ double max_f64(double a, double b) {
@@ -128,15 +122,6 @@ __device__ __forceinline__ bool meet(Meet *f, uint32_t cl, uint32_t n, double &f
     refined = (long long)(inc >> 32);
     return true;
 }
-
-// Lanes of the mask below this one.
-__device__ __forceinline__ int lanes_below(uint64_t mask) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-}
-
-// Flags of the edge list's entries.
-constexpr uint32_t LEAVES = 1u << 31, BOUNDARY = 1u << 30;
 
 // Four waves per SIMD (at most 128 VGPRs, a few spilled) outrun three
 // unspilled ones: the LDS of four 256-cell workgroups fits a CU.

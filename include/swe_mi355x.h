@@ -118,10 +118,18 @@ int swe_step(swe_handle *h, double dt, int forward, double *dt_cfl, int64_t *n_r
 int swe_run(swe_handle *h, int64_t n_steps, double dt0, int forward, double dt_clamp,
             double *time, double *dt_next);
 
+/* The device's null stream (whose hipStream_t is NULL) as a `stream` argument
+ * of swe_step_device, swe_forward_device, swe_adjoint_step_device,
+ * swe_adapt_record_device and their batch forms.  A caller whose own work is on
+ * the null stream names it so: the library's stream is ordered with it too,
+ * but each change from one to the other costs 25-30 us. */
+#define SWE_STREAM_NULL ((void *)1)
+
 /* Device-pointer step for callers that own device memory (the PyTorch
  * binding): reads eta/hu/hv/b at the given device addresses, writes
  * eta_out/hu_out/hv_out (must not alias the inputs), on `stream`
- * (a hipStream_t, NULL = the library's stream).  dt_cfl_dev and
+ * (a hipStream_t, NULL = the library's stream, SWE_STREAM_NULL = the device's
+ * null stream).  dt_cfl_dev and
  * n_refine_dev (nullable) are device scalars that receive the step's CFL
  * minimum and refinement count; refine_dev (nullable) receives the flags.
  * Asynchronous; calls on one handle must not overlap, whatever their streams. */
@@ -175,7 +183,8 @@ int swe_step_device_noalloc(const swe_device_mesh *mesh, const double *eta, cons
  * traversal Q^{n+1} = F(Q^n, b; dt_n) with dt_n and the wet/dry limiter
  * decisions frozen from the forward pass, swe_adjoint_step_device computes
  * lam^n = (dF/dQ^n)^T lam^{n+1} and adds (dF/db)^T lam^{n+1} to gb.
- * All pointers are device addresses; asynchronous on `stream`.
+ * All pointers are device addresses; asynchronous on `stream` (as for
+ * swe_step_device).
  *
  * swe_forward_device: one traversal on caller buffers with dt read from
  * device memory (*dt_dev), the CFL minimum written to *dt_cfl_dev (nullable)

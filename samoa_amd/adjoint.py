@@ -40,7 +40,7 @@ import math
 import numpy as np
 import torch
 
-from .swe import Batch, EulerTimestep, Mesh
+from .swe import STREAM_NULL, Batch, EulerTimestep, Mesh
 
 
 def _p(t: torch.Tensor) -> int:
@@ -126,7 +126,10 @@ class GaugeInversion:
         return torch.empty(self.n, dtype=torch.float64, device=self.device)
 
     def _stream(self):
-        return torch.cuda.current_stream(self.device).cuda_stream
+        """The current stream, so that the sweeps' kernels and torch's share
+        one: between torch's default stream and the handle's own, every change
+        waited 25-30 us (a step of a depth-15 sweep takes 10 us)."""
+        return torch.cuda.current_stream(self.device).cuda_stream or STREAM_NULL
 
     def _dt(self, step):
         return _p(self.dt) + 8 * self.n_scen * step
@@ -173,17 +176,18 @@ class GaugeInversion:
         """Forward sweep: gauge values after each step and the tape: every
         state and mask (store_all) or the checkpoints Q^{jK}."""
         q = [eta0.detach().contiguous().clone(), self._zeros(), self._zeros()]
-        series = torch.empty(self.n_steps, len(self.gauges), dtype=torch.float64, device=self.device)
         if self.store_all:
-            # every slot is written by a traversal before it is read
-            states = [q] + [[self._empty() for _ in range(3)] for _ in range(self.n_steps - 1)]
+            # every slot is written by a traversal before it is read; the
+            # elevations lie in one tensor, so one gather reads all gauges
+            etas = torch.empty(self.n_steps, self.n, dtype=torch.float64, device=self.device)
+            states = [q] + [[e, self._empty(), self._empty()] for e in etas]
             masks = torch.empty(self.n_steps, self.n, dtype=torch.int8, device=self.device)
-            last = [self._empty() for _ in range(3)]
             for n in range(self.n_steps):
-                out = states[n + 1] if n + 1 < self.n_steps else last
-                self._fwd(states[n], out, b, n, masks=masks[n])
-                torch.index_select(out[0], 0, self.gauges, out=series[n])
+                self._fwd(states[n], states[n + 1], b, n, masks=masks[n])
+            series = torch.index_select(etas, 1, self.gauges)
+            states.pop()
             return series, {"states": states, "masks": masks}
+        series = torch.empty(self.n_steps, len(self.gauges), dtype=torch.float64, device=self.device)
         out = [self._empty() for _ in range(3)]
         checkpoints = {}
         for n in range(self.n_steps):

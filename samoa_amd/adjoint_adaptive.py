@@ -87,7 +87,8 @@ class RemeshedRun:
             dtd = torch.tensor([dts[k]], dtype=torch.float64, device=self.device)
             masks = torch.empty(q[0].shape[0], dtype=torch.int8, device=self.device)
             self.op.forward_device(*map(P, q), *map(P, out), P(dtd), forward, masks=P(masks),
-                                   stream=torch.cuda.current_stream().cuda_stream)
+                                   stream=torch.cuda.current_stream().cuda_stream or
+                                   swe.STREAM_NULL)
             self.steps.append((m, dtd, forward, *q, masks))
             eta, hu, hv = (t.cpu().numpy() for t in out)
             outs.append((eta.copy(), hu.copy(), hv.copy(), b.copy()))

@@ -997,6 +997,13 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
 
 // Forward traversal on caller-owned device buffers (all scenarios), dt read
 // from device memory per scenario, limiter masks recorded (nullable).
+// The stream that a caller names: NULL the handle's, SWE_STREAM_NULL the
+// device's null stream.
+hipStream_t stream_of(const Batch &B, void *stream) {
+    if (stream == SWE_STREAM_NULL) return nullptr;
+    return stream ? (hipStream_t)stream : B.stream;
+}
+
 int batch_forward_device(Batch &B, const double *eta, const double *hu, const double *hv,
                          const double *b, double *eta_out, double *hu_out, double *hv_out,
                          const double *dt_dev, int forward, double *dt_cfl_dev, int8_t *masks,
@@ -1005,7 +1012,7 @@ int batch_forward_device(Batch &B, const double *eta, const double *hu, const do
         return fail(SWE_ERR_ARG, "forward_device: null argument");
     if (eta_out == eta || hu_out == hu || hv_out == hv)
         return fail(SWE_ERR_ARG, "forward_device: outputs must not alias inputs");
-    hipStream_t st = stream ? (hipStream_t)stream : B.stream;
+    hipStream_t st = stream_of(B, stream);
     swe::StepArgs a = make_args(B, 0, 1, forward);
     a.eta = eta;
     a.hu = hu;
@@ -1034,7 +1041,7 @@ int batch_adjoint_device(Batch &B, const double *eta, const double *hu, const do
         return fail(SWE_ERR_ARG, "adjoint_device: null argument");
     if (leta_out == leta || lhu_out == lhu || lhv_out == lhv)
         return fail(SWE_ERR_ARG, "adjoint_device: outputs must not alias inputs");
-    hipStream_t st = stream ? (hipStream_t)stream : B.stream;
+    hipStream_t st = stream_of(B, stream);
     swe::AdjArgs a{};
     a.eta = eta;
     a.hu = hu;
@@ -1245,7 +1252,7 @@ int swe_adapt_record_device(swe_handle *h, int8_t *code, int64_t *base, int64_t 
     if (b_sampled) *b_sampled = B.ad_record_sampled ? 1 : 0;
     if (!code && !base) return SWE_OK;
     if (!code || !base) return fail(SWE_ERR_ARG, "swe_adapt_record_device: code and base go together");
-    hipStream_t st = stream ? (hipStream_t)stream : B.stream;
+    hipStream_t st = stream_of(B, stream);
     if (B.ad_record_n < 0) {
         HIP_TRY(swe::identity_record(n, code, base, st));
     } else {
@@ -1316,7 +1323,7 @@ int swe_step_device(swe_handle *h, const double *eta, const double *hu, const do
     if (eta_out == eta || hu_out == hu || hv_out == hv)
         return fail(SWE_ERR_ARG, "swe_step_device: outputs must not alias inputs");
     Batch &B = h->B;
-    hipStream_t s = stream ? (hipStream_t)stream : B.stream;
+    hipStream_t s = stream_of(B, stream);
     swe::StepArgs a = make_args(B, 0, 1, forward);
     a.eta = eta;
     a.hu = hu;

@@ -30,6 +30,7 @@ BC_OUTFLOW = 0
 BC_WALL = 1
 ARITH_EXACT = 0        # every operation rounds as the reference's
 ARITH_TOLERANCED = 1   # shared reciprocals, refined estimates, within 1e-12 per step
+STREAM_NULL = 1  # the device's null stream, torch's default (0 names the handle's own)
 G = 9.80665  # SWE_data_types.f90:34
 
 

@@ -117,7 +117,7 @@ adjoint_step_kernel(AdjArgs args) {
             s_q[1][t] = qu;
             s_q[2][t] = qv;
             s_q[3][t] = qb;
-            const ClearCell cc = clear_cell(qe, qu, qv, qb, drytol, g);
+            const ClearCell cc = clear_cell<SOLVER>(qe, qu, qv, qb, drytol, g);
             s_x[0][t] = cc.r;
             s_x[1][t] = cc.c;
             s_mask[t] = (int8_t)mk;
@@ -246,7 +246,7 @@ adjoint_step_kernel(AdjArgs args) {
                 const double l0 = a.leta[x], l1 = a.lhu[x], l2 = a.lhv[x];
                 const int dl = sc.depth >= 0 ? sc.depth : a.depth[gt + o];
                 if (FIRST) {
-                    const ClearCell y = clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+                    const ClearCell y = clear_cell<SOLVER>(R[0], R[1], R[2], R[3], drytol, g);
                     R[4] = y.r;
                     R[5] = y.c;
                 }

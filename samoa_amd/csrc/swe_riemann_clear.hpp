@@ -41,17 +41,31 @@
 //
 // Divisions: a / b = fma(fma(-b, q, a), r, q), q = a r, with r the reciprocal
 // of b to within an ulp (the hardware estimate and two Newton steps): the
-// correctly rounded quotient (Markstein) as long as nothing under- or
-// overflows, so divisions by one value share one reciprocal, and a cell's is
-// computed once for its three edges.  What could under- or overflow is kept
-// out by clear_cell: a cell whose momenta or bathymetry are neither 0 nor in
-// [2^-240, 2^60], or whose depth is above 2^40, gets a NaN for c, which fails
-// the test on its edges.  A sum of doubles is 0 or at least the last place of
-// its smallest term, so on the others the rotated momenta are 0 or above
-// 2^-294, u (h < 2^40) above 2^-334, uL uR (hR - hL) above 2^-740 (clear
-// depths are above 2^-19), l2 times that above 2^-745, and the smallest
-// numerator, of beta1, above 2^-798: far from 2^-969, below which the
-// remainder fma(-b, q, a) would round.
+// correctly rounded quotient (Markstein) as long as nothing overflows and a is
+// 0 or at least 2^-969 (below, the remainder fma(-b, q, a) would round).
+// Divisions by one value share one reciprocal, and a cell's is computed once for
+// its three edges.  clear_cell keeps out what could overflow or get that small:
+// a cell whose momenta or bathymetry are neither 0 nor in [2^-N, 2^60], or
+// whose depth is above 2^40, gets a NaN for c, which fails the test on its
+// edges.  N = 740 for the augmented solver.  A sum of doubles is 0 or at least
+// the last place of its smallest term, and c > 0.06 means g h > 2^-9, so:
+//   - u's numerators (the rotated momenta) are 0 or above 2^-795, u above
+//     2^-835, uhat's numerator above 2^-893;
+//   - if the beds differ, delb > 2^-793 and deldelh's and deldelphi's numerators
+//     are above 2^-812.  delphi - deldelphi is 0 or above 2^-855, d0 above
+//     2^-847, and the numerators of beta0, beta1 and beta2 are 0 or above 2^-914;
+//   - if they do not, deldelh = deldelphi = 0, d0 = hR - hL, and where that is
+//     not 0 (then above 2^-73) it exceeds all that is tiny in a numerator.  At
+//     equal depths delphi = fl(delhu usum), and beta1's numerator may be anything
+//     small; but then f10 = beta0 r20 and f12, of size |delhu| > 2^-849 times
+//     l0^2 / span > 2^-34, exceed beta1 < 2^-966 by 2^80 and absorb it.
+// The f-wave solver's beta1 is not absorbed where beds are equal and depths differ
+// by less than the surface shows: there the numerator is uL uR (hR - hL), and
+// N = 340 keeps it above 2^-945.
+// (The momenta of a tsunami fall off as its source's Gaussian: with N = 240 for
+// both, up to all of the far ocean missed the short path, depending on the
+// source's width: over eight sources the d21 step took 144-200 us, now 145-150,
+// the d20 adjoint 113-213 us, now 112-117.)
 #pragma once
 
 #include "swe_riemann.hpp"
@@ -93,6 +107,7 @@ struct ClearCell {
 // takes the general path otherwise).
 constexpr double CLEAR_MIN_G = 0x1p-10, CLEAR_MAX_G = 0x1p10;
 
+template <int SOLVER>
 SWE_HD ClearCell clear_cell(double eta, double hu, double hv, double b, double drytol, double g) {
     const double h = eta - b;
     ClearCell k{0.0, 0.0};
@@ -118,7 +133,8 @@ SWE_HD ClearCell clear_cell(double eta, double hu, double hv, double b, double d
 #endif
     e = e < e1 ? e : e1;
     e = e < e2 ? e : e2;
-    const bool tame = e > -240 && fabs(hu) + fabs(hv) + fabs(b) < 0x1p60 && h < 0x1p40 && g_fits;
+    const bool tame = e > (SOLVER == 1 ? -340 : -740) && fabs(hu) + fabs(hv) + fabs(b) < 0x1p60 &&
+                      h < 0x1p40 && g_fits;
     if (!tame) k.c = __builtin_nan("");
     return k;
 }

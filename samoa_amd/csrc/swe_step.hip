@@ -252,7 +252,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
                 s_q[2][t] = vv;
                 s_q[3][t] = bb;
                 if constexpr (CLEAR) {
-                    const ClearCell k = clear_cell(e, u, vv, bb, drytol, g);
+                    const ClearCell k = clear_cell<SOLVER>(e, u, vv, bb, drytol, g);
                     s_x[0][t] = k.r;
                     s_x[1][t] = k.c;
                 }
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
                     R[4] = cq.sq;
                 }
                 if constexpr (SHORT && CLEAR) {
-                    const ClearCell x = clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+                    const ClearCell x = clear_cell<SOLVER>(R[0], R[1], R[2], R[3], drytol, g);
                     R[4] = x.r;
                     R[5] = x.c;
                 }

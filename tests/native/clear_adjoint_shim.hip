@@ -10,8 +10,8 @@ static void pairs(long n, const double *nrm, const double *L, const double *R, c
         for (int m = 0; m < 8; ++m) want[m] = got[m] = 0.0;
         swe::edge_flux_adj<SOLVER>(nrm[0], nrm[1], L[0], L[1], L[2], L[3], R[0], R[1], R[2], R[3],
                                    drytol, g, 1.0 / (16.0 * g), gfL, gfR, want, want + 4);
-        const swe::ClearCell a = swe::clear_cell(L[0], L[1], L[2], L[3], drytol, g);
-        const swe::ClearCell b = swe::clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+        const swe::ClearCell a = swe::clear_cell<SOLVER>(L[0], L[1], L[2], L[3], drytol, g);
+        const swe::ClearCell b = swe::clear_cell<SOLVER>(R[0], R[1], R[2], R[3], drytol, g);
         const double hL = L[0] - L[3], hR = R[0] - R[3];
         const swe::ClearEdge e =
             swe::clear_edge(nrm[0], nrm[1], hL, L[1], L[2], a.r, hR, R[1], R[2], b.r);

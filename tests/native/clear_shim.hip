@@ -11,8 +11,8 @@ static int both(const double *n, const double *L, const double *R, double drytol
                            1.0 / (16.0 * g), a, b);
     const double w[8] = {a.h, a.hu, a.hv, a.s, b.h, b.hu, b.hv, b.s};
     for (int i = 0; i < 8; ++i) want[i] = w[i];
-    const swe::ClearCell l = swe::clear_cell(L[0], L[1], L[2], L[3], drytol, g);
-    const swe::ClearCell r = swe::clear_cell(R[0], R[1], R[2], R[3], drytol, g);
+    const swe::ClearCell l = swe::clear_cell<SOLVER>(L[0], L[1], L[2], L[3], drytol, g);
+    const swe::ClearCell r = swe::clear_cell<SOLVER>(R[0], R[1], R[2], R[3], drytol, g);
     const double hL = L[0] - L[3], hR = R[0] - R[3];
     const swe::ClearEdge e =
         swe::clear_edge(n[0], n[1], hL, L[1], L[2], l.r, hR, R[1], R[2], r.r);

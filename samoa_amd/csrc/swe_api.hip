@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -16,6 +17,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -194,6 +196,47 @@ int pack_mesh(const swe_mesh_desc &d, const double *normal, std::vector<int32_t>
 
 }  // namespace
 
+// Pinned staging of transfers (transfer below).
+constexpr int STAGE_PARTS = 4;
+constexpr size_t STAGE_LEAST = 64 << 10, STAGE_SMALL = 2 << 20;
+constexpr size_t RING_SLOTS = 8, RING_PIECE = 1 << 20, RING_MIN = 4 << 20;
+
+// Pinned buffers of the three sizes, kept from closed handles for new ones
+// (pinning 64 KB takes 60 us, 8 MB 200 us): at most four of each, 40 MB.
+constexpr size_t STAGE_SIZES[3] = {STAGE_LEAST, STAGE_SMALL, RING_SLOTS * RING_PIECE};
+constexpr int STAGE_KEPT = 4;
+std::mutex g_stage_mutex;
+char *g_stage_free[3][STAGE_KEPT];
+int g_stage_count[3];
+
+// A buffer of STAGE_SIZES[k], usable from every device; null if there is none.
+char *stage_take(int k) {
+    {
+        std::lock_guard<std::mutex> lock(g_stage_mutex);
+        if (g_stage_count[k] > 0) return g_stage_free[k][--g_stage_count[k]];
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, STAGE_SIZES[k], hipHostMallocCoherent | hipHostMallocPortable) !=
+        hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return (char *)p;
+}
+
+// Gives back a buffer that no queued work uses.
+void stage_give(int k, char *p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lock(g_stage_mutex);
+        if (g_stage_count[k] < STAGE_KEPT) {
+            g_stage_free[k][g_stage_count[k]++] = p;
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 struct Batch {
     int device = 0;
     hipStream_t stream = nullptr;      // where work is launched (caller may replace it)
@@ -211,6 +254,9 @@ struct Batch {
     int32_t *d_chunk_scen = nullptr;
     swe::Slots *d_slots = nullptr;
     double *d_dt = nullptr;  // [nscen] host-chosen dt per scenario
+    char *stage = nullptr;   // pinned, STAGE_SIZES[stage_size], taken when a transfer needs it
+    int stage_size = 0;
+    hipEvent_t ring_event[RING_SLOTS] = {};
     double *d_part_max[2] = {nullptr, nullptr};  // [part_cap] fastest cell per chunk
     int32_t *d_part_nref = nullptr;   // [part_cap] refinement count per chunk
     // A chain of steps without finalize kernels (batch_run): the device dt is
@@ -311,6 +357,9 @@ void release(Batch &B) {
     (void)hipFree(B.ad_eslot);
     (void)hipFree(B.raster);
     if (B.ad_host) (void)hipHostFree(B.ad_host);
+    stage_give(B.stage_size, B.stage);
+    for (auto &e : B.ring_event)
+        if (e) (void)hipEventDestroy(e);
     if (B.own_stream) (void)hipStreamDestroy(B.own_stream);
 }
 
@@ -521,17 +570,207 @@ swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
     return a;
 }
 
+// Transfers between device memory and the caller's arrays, through a pinned
+// buffer of the handle that a kernel reads and writes.
+//
+// Small ones: a copy to or from pageable memory costs 12-20 us whatever its size,
+// and a call needs up to five.  One launch moves all parts, then the host
+// copies (or before, to the device).  A d8 host loop (512 cells; traversal with
+// flags, download): 42 + 60 -> 24 + 17 us; up to STAGE_SMALL the kernel's way is
+// no slower in either direction (us, direct / staged: 1 MB down 79 / 58, up
+// 63 / 51; 2 MB 124 / 101, 83 / 84; 4 MB 240 / 233, 135 / 156).
+struct Part {
+    void *dev, *host;
+    size_t bytes;
+    bool packed = false;  // to the host: neighbours (o << 2) | back edge, wanted as o
+};
+
+struct StageArgs {
+    char *dev[STAGE_PARTS], *stage[STAGE_PARTS];
+    uint32_t bytes[STAGE_PARTS];
+    int to_host;
+    int packed;  // bit p: part p is packed
+};
+
+__host__ __device__ inline int32_t unpack_nbr(int32_t p) { return p < 0 ? -1 : p >> 2; }
+
+// Part blockIdx.y, eight bytes a thread (parts start on eight bytes), its
+// last bytes singly.
+__global__ __launch_bounds__(256) void stage_kernel(StageArgs a) {
+    const int p = blockIdx.y;
+    const uint32_t n = a.bytes[p], i = blockIdx.x * 256 + threadIdx.x, words = n / 8;
+    const char *const src = a.to_host ? a.dev[p] : a.stage[p];
+    char *const dst = a.to_host ? a.stage[p] : a.dev[p];
+    if (a.packed >> p & 1) {  // whole int32
+        const int32_t *const s = reinterpret_cast<const int32_t *>(src);
+        int32_t *const d = reinterpret_cast<int32_t *>(dst);
+        if (i < words) reinterpret_cast<int2 *>(d)[i] = {unpack_nbr(s[2 * i]), unpack_nbr(s[2 * i + 1])};
+        else if (i == words && n % 8) d[2 * i] = unpack_nbr(s[2 * i]);
+    } else if (i < words) {
+        reinterpret_cast<uint64_t *>(dst)[i] = reinterpret_cast<const uint64_t *>(src)[i];
+    } else if (i < words + n % 8) {
+        const uint32_t k = words * 8 + (i - words);
+        dst[k] = src[k];
+    }
+}
+
+hipError_t launch_stage(const StageArgs &a, int parts, uint32_t longest, hipStream_t st) {
+    const unsigned blocks = (longest / 8 + 7 + 255) / 256;
+    hipLaunchKernelGGL(stage_kernel, dim3(blocks, (unsigned)parts), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+// The handle's pinned buffer, of at least `bytes` (no more than the ring's);
+// null: the copies go directly.
+char *stage_of(Batch &B, size_t bytes) {
+    if (B.stage && bytes <= STAGE_SIZES[B.stage_size]) return B.stage;
+    stage_give(B.stage_size, B.stage);  // every transfer waits for its launches
+    B.stage_size = bytes <= STAGE_LEAST ? 0 : (bytes <= STAGE_SMALL ? 1 : 2);
+    return B.stage = stage_take(B.stage_size);
+}
+
+// Large downloads: the host's copies into the caller's arrays (and the page
+// faults of new ones) are what takes the time, so threads share them, piece by
+// piece, while the kernel fills the other slots of the ring.  Direct / ring
+// with no, one and three more threads (us, arrays that had been written before):
+//     4.2 MB 244 / 220 / 177 / 194     16.8 MB 986 / 774 / 554 / 471
+//     8.4 MB 493 / 392 / 272 / 292     134 MB 7790 / 5527 / 5002 / 3059
+// (seven threads with pieces of half the size: 237, 362, 587, 3724).
+int download_ring(Batch &B, const Part *parts, int count) {
+    struct Piece {
+        char *dev, *host;
+        uint32_t bytes;
+        bool packed;
+    };
+    std::vector<Piece> pieces;
+    for (int i = 0; i < count; ++i)
+        for (size_t o = 0; o < parts[i].bytes; o += RING_PIECE) {
+            const size_t n = parts[i].bytes - o < RING_PIECE ? parts[i].bytes - o : RING_PIECE;
+            pieces.push_back({(char *)parts[i].dev + o, (char *)parts[i].host + o, (uint32_t)n,
+                              parts[i].packed});
+        }
+    const size_t n = pieces.size();
+    std::vector<std::atomic<char>> copied(n);
+    for (auto &c : copied) c = 0;
+    std::atomic<size_t> next{0}, launched{0};
+    std::atomic<int> error{0};
+    for (auto &e : B.ring_event)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    const int device = B.device;
+    // copies pieces as they arrive, until none is left
+    auto copier = [&](bool other_thread) {
+        if (other_thread && hipSetDevice(device) != hipSuccess) error = 1;
+        for (size_t k; (k = next++) < n;) {
+            while (launched <= k && !error) std::this_thread::yield();
+            if (!error && hipEventSynchronize(B.ring_event[k % RING_SLOTS]) != hipSuccess) error = 1;
+            if (!error)
+                memcpy(pieces[k].host, B.stage + k % RING_SLOTS * RING_PIECE, pieces[k].bytes);
+            copied[k] = 1;
+        }
+    };
+    std::vector<std::thread> threads;
+    try {
+        const int helpers = n < 12 ? 1 : 3;
+        for (int i = 0; i < helpers; ++i) threads.emplace_back(copier, true);
+    } catch (...) {  // fewer threads then
+    }
+    hipError_t e = hipSuccess;
+    for (size_t k = 0; k < n && !error; ++k) {
+        if (k >= RING_SLOTS) {
+            if (threads.empty()) {
+                // alone: copy what has been launched
+                const size_t c = next++;
+                e = hipEventSynchronize(B.ring_event[c % RING_SLOTS]);
+                if (e != hipSuccess) break;
+                memcpy(pieces[c].host, B.stage + c % RING_SLOTS * RING_PIECE, pieces[c].bytes);
+                copied[c] = 1;
+            }
+            while (!copied[k - RING_SLOTS] && !error) std::this_thread::yield();
+        }
+        StageArgs a{};
+        a.dev[0] = pieces[k].dev;
+        a.stage[0] = B.stage + k % RING_SLOTS * RING_PIECE;
+        a.bytes[0] = pieces[k].bytes;
+        a.to_host = 1;
+        a.packed = pieces[k].packed ? 1 : 0;
+        e = launch_stage(a, 1, a.bytes[0], B.stream);
+        if (e == hipSuccess) e = hipEventRecord(B.ring_event[k % RING_SLOTS], B.stream);
+        if (e != hipSuccess) break;
+        launched = k + 1;
+    }
+    if (e != hipSuccess) error = 1;
+    copier(false);
+    for (auto &t : threads) t.join();
+    if (e != hipSuccess || error) {
+        B.stage = nullptr;  // launches may still write to it: not given back
+        return fail(SWE_ERR_HIP, "download: %s", e != hipSuccess ? hipGetErrorString(e) : "copying");
+    }
+    HIP_TRY(hipStreamSynchronize(B.stream));
+    return SWE_OK;
+}
+
+// Moves the parts (those of no bytes are skipped) and waits for them, after
+// what is queued on the handle's stream.
+int transfer(Batch &B, const Part *parts, int count, bool to_host) {
+    StageArgs a{};
+    const Part *from[STAGE_PARTS];
+    size_t total = 0, longest = 0;
+    int n = 0;
+    for (int i = 0; i < count; ++i) total += (parts[i].bytes + 7) / 8 * 8;
+    const bool ring = to_host && total >= RING_MIN;
+    char *stage = nullptr;
+    if (ring || total <= STAGE_SMALL) stage = stage_of(B, ring ? RING_SLOTS * RING_PIECE : total);
+    if (ring && stage) return download_ring(B, parts, count);
+    if (!stage) {
+        for (int i = 0; i < count; ++i) {
+            if (!parts[i].bytes) continue;
+            if (to_host)
+                HIP_TRY(hipMemcpyAsync(parts[i].host, parts[i].dev, parts[i].bytes,
+                                       hipMemcpyDeviceToHost, B.stream));
+            else
+                HIP_TRY(hipMemcpyAsync(parts[i].dev, parts[i].host, parts[i].bytes,
+                                       hipMemcpyHostToDevice, B.stream));
+        }
+        HIP_TRY(hipStreamSynchronize(B.stream));
+        for (int i = 0; i < count; ++i) {
+            int32_t *const v = (int32_t *)parts[i].host;
+            if (parts[i].packed)
+                for (size_t k = 0; k < parts[i].bytes / sizeof(int32_t); ++k) v[k] = unpack_nbr(v[k]);
+        }
+        return SWE_OK;
+    }
+    total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!parts[i].bytes) continue;
+        a.dev[n] = (char *)parts[i].dev;
+        a.stage[n] = stage + total;
+        a.bytes[n] = (uint32_t)parts[i].bytes;
+        a.packed |= parts[i].packed ? 1 << n : 0;
+        longest = parts[i].bytes > longest ? parts[i].bytes : longest;
+        total += (parts[i].bytes + 7) / 8 * 8;
+        from[n++] = &parts[i];
+    }
+    a.to_host = to_host ? 1 : 0;
+    if (!to_host)
+        for (int k = 0; k < n; ++k) memcpy(a.stage[k], from[k]->host, from[k]->bytes);
+    if (n > 0) HIP_TRY(launch_stage(a, n, (uint32_t)longest, B.stream));
+    HIP_TRY(hipStreamSynchronize(B.stream));
+    if (to_host)
+        for (int k = 0; k < n; ++k) memcpy(from[k]->host, a.stage[k], from[k]->bytes);
+    return SWE_OK;
+}
+
 int batch_upload(Batch &B, int32_t s, const double *eta, const double *hu, const double *hv,
                  const double *b) {
     if (s < 0 || s >= B.nscen) return fail(SWE_ERR_ARG, "scenario %d out of range", s);
     if (!eta || !hu || !hv || !b) return fail(SWE_ERR_ARG, "upload: null argument");
     const size_t bytes = sizeof(double) * (size_t)B.scen[s].n;
     const int64_t o = B.scen[s].cell_off;
-    HIP_TRY(hipMemcpyAsync(B.eta[B.cur] + o, eta, bytes, hipMemcpyHostToDevice, B.stream));
-    HIP_TRY(hipMemcpyAsync(B.hu[B.cur] + o, hu, bytes, hipMemcpyHostToDevice, B.stream));
-    HIP_TRY(hipMemcpyAsync(B.hv[B.cur] + o, hv, bytes, hipMemcpyHostToDevice, B.stream));
-    HIP_TRY(hipMemcpyAsync(B.b + o, b, bytes, hipMemcpyHostToDevice, B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
+    const Part parts[4] = {{B.eta[B.cur] + o, (void *)eta, bytes},
+                           {B.hu[B.cur] + o, (void *)hu, bytes},
+                           {B.hv[B.cur] + o, (void *)hv, bytes},
+                           {B.b + o, (void *)b, bytes}};
+    SWE_TRY(transfer(B, parts, 4, false));
     B.uploaded[s] = 1;
     B.flags_valid = false;
     return SWE_OK;
@@ -542,12 +781,11 @@ int batch_download(Batch &B, int32_t s, double *eta, double *hu, double *hv, dou
     if (!B.uploaded[s]) return fail(SWE_ERR_STATE, "download: scenario %d has no state", s);
     const size_t bytes = sizeof(double) * (size_t)B.scen[s].n;
     const int64_t o = B.scen[s].cell_off;
-    if (eta) HIP_TRY(hipMemcpyAsync(eta, B.eta[B.cur] + o, bytes, hipMemcpyDeviceToHost, B.stream));
-    if (hu) HIP_TRY(hipMemcpyAsync(hu, B.hu[B.cur] + o, bytes, hipMemcpyDeviceToHost, B.stream));
-    if (hv) HIP_TRY(hipMemcpyAsync(hv, B.hv[B.cur] + o, bytes, hipMemcpyDeviceToHost, B.stream));
-    if (b) HIP_TRY(hipMemcpyAsync(b, B.b + o, bytes, hipMemcpyDeviceToHost, B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
-    return SWE_OK;
+    const Part parts[4] = {{B.eta[B.cur] + o, eta, eta ? bytes : 0},
+                           {B.hu[B.cur] + o, hu, hu ? bytes : 0},
+                           {B.hv[B.cur] + o, hv, hv ? bytes : 0},
+                           {B.b + o, b, b ? bytes : 0}};
+    return transfer(B, parts, 4, true);
 }
 
 // The meeting points of a step of few chunks per scenario, else null.
@@ -562,20 +800,21 @@ int batch_step(Batch &B, const double *dt, int forward, double *dt_cfl, int64_t 
                int8_t *refine_host) {
     if (!dt || !dt_cfl) return fail(SWE_ERR_ARG, "step: null argument");
     if (!all_uploaded(B)) return fail(SWE_ERR_STATE, "step: not every scenario has a state");
-    HIP_TRY(hipMemcpyAsync(B.d_dt, dt, sizeof(double) * (size_t)B.nscen, hipMemcpyHostToDevice,
-                           B.stream));
     swe::StepArgs a = make_args(B, B.cur, 1 - B.cur, forward);
-    a.dt_host = B.d_dt;
+    if (B.nscen == 1) {
+        a.dt = dt[0];
+    } else {
+        HIP_TRY(hipMemcpyAsync(B.d_dt, dt, sizeof(double) * (size_t)B.nscen,
+                               hipMemcpyHostToDevice, B.stream));
+        a.dt_host = B.d_dt;
+    }
     a.meet = meet_of(B);
     a.refine = (refine_host || B.keep_flags) ? B.refine : nullptr;
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, B.stream));
     std::vector<swe::Slots> res((size_t)B.nscen);
-    HIP_TRY(hipMemcpyAsync(res.data(), B.d_slots, sizeof(swe::Slots) * res.size(),
-                           hipMemcpyDeviceToHost, B.stream));
-    if (refine_host)
-        HIP_TRY(hipMemcpyAsync(refine_host, B.refine, (size_t)B.ncells, hipMemcpyDeviceToHost,
-                               B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
+    const Part parts[2] = {{B.d_slots, res.data(), sizeof(swe::Slots) * res.size()},
+                           {B.refine, refine_host, refine_host ? (size_t)B.ncells : 0}};
+    SWE_TRY(transfer(B, parts, 2, true));
     for (int32_t s = 0; s < B.nscen; ++s) {
         dt_cfl[s] = res[s].res_dtcfl;
         if (n_refine) n_refine[s] = (int64_t)res[s].res_nref;
@@ -702,9 +941,8 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     if (!time && !dt_next) return SWE_OK;
     SWE_TRY(chain_flush(B));
     std::vector<swe::Slots> res((size_t)B.nscen);
-    HIP_TRY(hipMemcpyAsync(res.data(), B.d_slots, sizeof(swe::Slots) * res.size(),
-                           hipMemcpyDeviceToHost, B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
+    const Part part{B.d_slots, res.data(), sizeof(swe::Slots) * res.size()};
+    SWE_TRY(transfer(B, &part, 1, true));
     for (int32_t s = 0; s < B.nscen; ++s) {
         if (time) time[s] = res[s].time;
         if (dt_next) dt_next[s] = res[s].dt;
@@ -1279,16 +1517,10 @@ int swe_download_mesh(swe_handle *h, int8_t *depth, int8_t *plotter, int32_t *nb
     Batch &B = h->B;
     if (B.nscen != 1) return fail(SWE_ERR_ARG, "swe_download_mesh: a batch has no single mesh");
     const int64_t n = B.ncells;
-    if (depth) HIP_TRY(hipMemcpyAsync(depth, B.depth, (size_t)n, hipMemcpyDeviceToHost, B.stream));
-    if (plotter)
-        HIP_TRY(hipMemcpyAsync(plotter, B.plotter, (size_t)n, hipMemcpyDeviceToHost, B.stream));
-    if (nbr)
-        HIP_TRY(hipMemcpyAsync(nbr, B.nbr, sizeof(int32_t) * 3 * (size_t)n, hipMemcpyDeviceToHost,
-                               B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
-    if (nbr)  // (o << 2) | back edge -> o
-        for (int64_t i = 0; i < 3 * n; ++i) nbr[i] = nbr[i] < 0 ? -1 : (nbr[i] >> 2);
-    return SWE_OK;
+    const Part parts[3] = {{B.depth, depth, depth ? (size_t)n : 0},
+                           {B.plotter, plotter, plotter ? (size_t)n : 0},
+                           {B.nbr, nbr, nbr ? sizeof(int32_t) * 3 * (size_t)n : 0, true}};
+    return transfer(B, parts, 3, true);
 }
 
 int swe_set_stream(swe_handle *h, void *stream) {

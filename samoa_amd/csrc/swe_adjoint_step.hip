@@ -54,9 +54,7 @@ adjoint_step_kernel(AdjArgs args) {
     __shared__ double s_seed[3][CH];  // s * lam^{n+1} after the limiter (per cell)
     __shared__ double s_gb[CH];       // each cell's b gradient so far
     __shared__ double s_g[4][3][CH];  // transpose-flux contributions per (edge, cell)
-    // The edges to solve, as in the step kernel: those inside the chunk, then
-    // those leaving it, then the packed neighbours of the latter.
-    __shared__ uint32_t s_list[3 * CH + 4];
+    __shared__ uint32_t s_list[3 * CH + 4];  // the edge list (swe_device.hpp)
     __shared__ uint16_t s_rest[3 * CH];  // entries left to the general solver
     __shared__ int8_t s_dep[CH], s_mask[CH];
     __shared__ int s_wsum[CH / 64], s_nrest;
@@ -80,7 +78,6 @@ adjoint_step_kernel(AdjArgs args) {
         // and what follows from t is computed where it is used: LDS addresses
         // kept across the loops are registers that the general solver lacks
         asm volatile("" : "+v"(t));
-        const int lane = t & 63, wave = t >> 6;
         // raised wave priority for the chunk's loads and edge list, as in the
         // forward step kernel
         __builtin_amdgcn_s_setprio(2);
@@ -93,9 +90,25 @@ adjoint_step_kernel(AdjArgs args) {
         const double g = a.g, drytol = sc.drytol, S = sc.scaling;
         const double dt = a.dt_dev ? scalar(a.dt_dev)[s] : a.dt;
 
-        // transpose of the cell update for this thread's cell
+        const uint32_t *const list =
+            a.lists ? a.lists + (uint64_t)chunk * list_words(CH) : nullptr;
+
+        // the stored list, or this thread's cell's neighbours to build it from
         int32_t nb[3] = {-1, -1, -1};
         int plot = 1;
+        uint32_t head = 0;
+        ListAhead<CH, CH> ahead;
+        if (list) {
+            head = scalar(list)[0];
+            ahead.load(list, t);
+        } else if (active) {
+            const int32_t *const nbr = a.nbr + 3 * (gt + lbase);
+            nb[0] = nbr[3 * t];
+            nb[1] = nbr[3 * t + 1];
+            nb[2] = nbr[3 * t + 2];
+            plot = a.plotter[gt + lbase + t];
+        }
+        // transpose of the cell update for this thread's cell
         if (active) {
             // every load in one round: the state, topology, masks and
             // adjoint inputs first, the depth (behind a branch) last
@@ -106,11 +119,6 @@ adjoint_step_kernel(AdjArgs args) {
             // only this cell's thread adds to its b gradient: read now, with
             // the other loads, not after the edge loop
             s_gb[t] = a.gb[x];
-            const int32_t *const nbr = a.nbr + 3 * (gt + lbase);
-            nb[0] = nbr[3 * t];
-            nb[1] = nbr[3 * t + 1];
-            nb[2] = nbr[3 * t + 2];
-            plot = a.plotter[gt + lbase + t];
             const int dep = sc.depth >= 0 ? sc.depth : (int)a.depth[gt + lbase + t];
             s_dep[t] = (int8_t)dep;
             s_q[0][t] = qe;
@@ -130,56 +138,16 @@ adjoint_step_kernel(AdjArgs args) {
         }
         if (t == 0) s_nrest = 0;
 
-        // Edges this thread's cell must solve: those leaving the chunk, and
-        // the inner ones whose other cell the traversal visits later (so from
-        // their left side).
-        int inner = 0, leave = 0;
-        if (active) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int32_t p = nb[k];
-                const int lo = (p >> 2) - lbase;  // chunk-local neighbour
-                if (!(p >= 0 && (uint32_t)lo < (uint32_t)cnt)) leave |= 1 << k;
-                else if (a.forward ? lo > t : lo < t) inner |= 1 << k;
-            }
-        }
-        // workgroup exclusive prefixes of both counts (0..3 each) via ballots,
-        // packed: inner in the low half, leaving in the high half
-        const int nin = __popc(inner), nout = __popc(leave);
-        const uint64_t i0 = __ballot(nin & 1), i1 = __ballot(nin & 2);
-        const uint64_t o0 = __ballot(nout & 1), o1 = __ballot(nout & 2);
-        const int wpre = lanes_below(i0) + 2 * lanes_below(i1) +
-                         ((lanes_below(o0) + 2 * lanes_below(o1)) << 16);
-        if (lane == 0)
-            s_wsum[wave] = __popcll(i0) + 2 * __popcll(i1) +
-                           ((__popcll(o0) + 2 * __popcll(o1)) << 16);
+        const int2 entries =
+            list ? ahead.put(list, head, t, s_list)
+                 : list_edges<CH, false>(
+                       t, cnt, lbase, nb, plot, s_wsum, [&](int k, int) { return nb[k] & 3; },
+                       [&](int i, uint32_t ent) { s_list[i] = ent; });
+        const int n_inner = entries.x, total = entries.y;
         __syncthreads();
-        int pre = wpre, sum = 0;
-#pragma unroll
-        for (int w = 0; w < CH / 64; ++w) {
-            const int ws = s_wsum[w];
-            pre += w < wave ? ws : 0;
-            sum += ws;
-        }
-        const int n_inner = sum & 0xffff, total = n_inner + (sum >> 16);
-        int pi = pre & 0xffff, po = n_inner + (pre >> 16);
-        const int turn = plot < 0 ? -plot : plot;  // edge normals: see the step kernel
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int d0 = k == 1 ? 1 : ((k == 0) == (plot > 0) ? 4 : 6);
-            const int32_t p = nb[k];
-            const bool in = inner & (1 << k), out = leave & (1 << k);
-            const uint32_t other =
-                in ? ((uint32_t)((p >> 2) - lbase) << 11) | ((uint32_t)(p & 3) << 20)
-                   : LEAVES | (p < 0 ? BOUNDARY : 0u);
-            if (in || out)
-                s_list[in ? pi : po] = (uint32_t)t | ((uint32_t)k << 9) |
-                                       ((uint32_t)((turn + d0) & 7) << 22) | other;
-            if (out) s_list[po + total - n_inner] = (uint32_t)p;
-            pi += in ? 1 : 0;
-            po += out ? 1 : 0;
-        }
-        __syncthreads();
+        // inner edges from their left side, as in the step kernel
+        const int left = a.forward ? 0 : 11, right = 11 - left;
+        const uint32_t opposite = a.forward ? 0u : 4u;
 
         __builtin_amdgcn_s_setprio(0);
         // One pass over the list (FIRST, clear_flux_adj; it lists the edges
@@ -196,7 +164,9 @@ adjoint_step_kernel(AdjArgs args) {
         for (int i = t; i < n; i += CH) {
             const int e = FIRST ? i : s_rest[i];
             const uint32_t ent = s_list[e];
-            const int lc = ent & 511, k = (ent >> 9) & 3, dir = (ent >> 22) & 7;
+            const bool inside = !(ent & LEAVES);
+            const int lc = (ent >> left) & 511, k = (ent >> (left + 9)) & 3;
+            const uint32_t dir = ((ent >> 22) & 7) ^ (inside ? opposite : 0u);
             double nx = s_dir[dir][0], ny = s_dir[dir][1];
             // both cells' state, 1/h and c, and seeds: left and right for an
             // inner edge; one that leaves the chunk may need them exchanged
@@ -211,8 +181,7 @@ adjoint_step_kernel(AdjArgs args) {
             }
 #pragma unroll
             for (int m = 0; m < 3; ++m) fL[m] = s_seed[m][lc] * len;
-            const bool inside = !(ent & LEAVES);
-            const int lo = (ent >> 11) & 511, ko = (ent >> 20) & 3;
+            const int lo = (ent >> right) & 511, ko = (ent >> (right + 9)) & 3;
             bool flip = false;
             if (inside) {
 #pragma unroll

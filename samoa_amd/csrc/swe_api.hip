@@ -237,6 +237,9 @@ void stage_give(int k, char *p) {
     (void)hipHostFree(p);
 }
 
+// Traversals of a changed mesh after which its edge lists are stored.
+constexpr int64_t LISTS_FROM = 2;
+
 struct Batch {
     int device = 0;
     hipStream_t stream = nullptr;      // where work is launched (caller may replace it)
@@ -248,6 +251,10 @@ struct Batch {
     std::vector<swe::Scen> scen;
     std::vector<int> uniform_depth;
     int64_t ncells = 0, ntopo = 0, nchunks = 0;
+    uint32_t *d_lists = nullptr;  // the chunks' edge lists (lists_valid), of lists_cap bytes
+    size_t lists_cap = 0;
+    bool lists_valid = false;
+    int64_t list_uses = 0;  // traversals since the mesh or the chunks changed
     int chunk = swe::DEFAULT_CHUNK;
     int64_t grid = 0;
     swe::Scen *d_scen = nullptr;
@@ -341,6 +348,7 @@ void release(Batch &B) {
     (void)hipFree(B.d_part_max[1]);
     (void)hipFree(B.d_part_nref);
     (void)hipFree(B.d_meet);
+    (void)hipFree(B.d_lists);
     (void)hipFree(B.b2);
     (void)hipFree(B.nbr2);
     (void)hipFree(B.plotter2);
@@ -386,6 +394,15 @@ int chain_flush(Batch &B) {
 // chunk -> scenario map (not needed for a single scenario).
 // upload = false: the device copy of the scenario table is already
 // current (the remesher's emit kernel wrote it).
+void drop_graphs(Batch &B) {
+    for (auto &row : B.graph)
+        for (GraphCache &gc : row)
+            if (gc.exec) {
+                (void)hipGraphExecDestroy(gc.exec);
+                gc = GraphCache{};
+            }
+}
+
 int rebuild_chunks(Batch &B, bool upload = true) {
     int64_t off = 0;
     for (auto &s : B.scen) {
@@ -427,12 +444,42 @@ int rebuild_chunks(Batch &B, bool upload = true) {
     if (upload)
         HIP_TRY(hipMemcpyAsync(B.d_scen, B.scen.data(), sizeof(swe::Scen) * B.scen.size(),
                                hipMemcpyHostToDevice, B.stream));
-    for (auto &row : B.graph)
-        for (GraphCache &gc : row)
-            if (gc.exec) {
-                (void)hipGraphExecDestroy(gc.exec);
-                gc = GraphCache{};
-            }
+    drop_graphs(B);
+    B.lists_valid = false;
+    B.list_uses = 0;
+    return SWE_OK;
+}
+
+// Stores the chunks' edge lists, on the handle's stream, and waits for them:
+// from then on any stream's steps may read them.  A mesh keeps its lists until
+// it or the chunk size changes.  Without the memory for them, steps build
+// their own.
+int store_lists(Batch &B) {
+    if (B.lists_valid) return SWE_OK;
+    const size_t bytes = swe::edge_list_bytes(B.nchunks, B.chunk);
+    if (bytes > B.lists_cap) {
+        (void)hipFree(B.d_lists);
+        B.d_lists = nullptr;
+        B.lists_cap = 0;
+        if (hipMalloc(&B.d_lists, bytes + bytes / 8) != hipSuccess) {
+            B.d_lists = nullptr;
+            (void)hipGetLastError();
+            return SWE_OK;
+        }
+        B.lists_cap = bytes + bytes / 8;
+    }
+    drop_graphs(B);  // captured without lists
+    HIP_TRY(swe::build_edge_lists(make_args(B, 0, 1, 1), B.chunk, B.d_lists, B.stream));
+    HIP_TRY(hipStreamSynchronize(B.stream));
+    B.lists_valid = true;
+    return SWE_OK;
+}
+
+// Before `steps` traversals of the handle's state: a changed mesh is worth its
+// lists once several traversals use them (building takes about what two save).
+int lists_for(Batch &B, int64_t steps) {
+    B.list_uses += steps;
+    if (!B.lists_valid && B.list_uses > LISTS_FROM) SWE_TRY(store_lists(B));
     return SWE_OK;
 }
 
@@ -536,7 +583,8 @@ int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
     HIP_TRY(hipMemset(B.d_meet, 0, sizeof(swe::Meet) * swe::MEET_SLOTS * (size_t)nscen));
     B.uploaded.assign((size_t)nscen, 0);
     B.cap = B.ncells;
-    return rebuild_chunks(B);
+    SWE_TRY(rebuild_chunks(B));
+    return store_lists(B);
 }
 
 swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
@@ -554,6 +602,7 @@ swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
     a.scen = B.d_scen;
     a.scen0 = B.scen[0];  // read in place of the table when it is the only one
     a.chunk_scen = B.d_chunk_scen;
+    a.lists = B.lists_valid ? B.d_lists : nullptr;
     a.slots = B.d_slots;
     a.part_max = B.d_part_max[1 - B.pp];  // not the one a chain may still need
     a.part_nref = B.d_part_nref;
@@ -800,6 +849,7 @@ int batch_step(Batch &B, const double *dt, int forward, double *dt_cfl, int64_t 
                int8_t *refine_host) {
     if (!dt || !dt_cfl) return fail(SWE_ERR_ARG, "step: null argument");
     if (!all_uploaded(B)) return fail(SWE_ERR_STATE, "step: not every scenario has a state");
+    SWE_TRY(lists_for(B, 1));
     swe::StepArgs a = make_args(B, B.cur, 1 - B.cur, forward);
     if (B.nscen == 1) {
         a.dt = dt[0];
@@ -855,6 +905,7 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
                                hipMemcpyHostToDevice, B.stream));
     }
 
+    SWE_TRY(lists_for(B, n_steps));
     // Meshes of few chunks step in a chain: a step forms its dt from the
     // partials of the one before, and a finalize kernel runs only for who
     // reads the results.
@@ -1233,8 +1284,6 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
     return SWE_OK;
 }
 
-// Forward traversal on caller-owned device buffers (all scenarios), dt read
-// from device memory per scenario, limiter masks recorded (nullable).
 // The stream that a caller names: NULL the handle's, SWE_STREAM_NULL the
 // device's null stream.
 hipStream_t stream_of(const Batch &B, void *stream) {
@@ -1242,6 +1291,8 @@ hipStream_t stream_of(const Batch &B, void *stream) {
     return stream ? (hipStream_t)stream : B.stream;
 }
 
+// Forward traversal on caller-owned device buffers (all scenarios), dt read
+// from device memory per scenario, limiter masks recorded (nullable).
 int batch_forward_device(Batch &B, const double *eta, const double *hu, const double *hv,
                          const double *b, double *eta_out, double *hu_out, double *hv_out,
                          const double *dt_dev, int forward, double *dt_cfl_dev, int8_t *masks,
@@ -1299,6 +1350,7 @@ int batch_adjoint_device(Batch &B, const double *eta, const double *hu, const do
     a.scen = B.d_scen;
     a.chunk_scen = B.d_chunk_scen;
     a.nchunks = B.nchunks;
+    a.lists = B.lists_valid ? B.d_lists : nullptr;
     a.dt_dev = dt_dev;
     a.g = B.g;
     a.inv16g = 1.0 / (16.0 * B.g);
@@ -1337,6 +1389,7 @@ int batch_set_tuning(Batch &B, int chunk, int64_t grid) {
     if (chunk != B.chunk) {
         B.chunk = chunk;
         SWE_TRY(rebuild_chunks(B));
+        SWE_TRY(store_lists(B));
     }
     return SWE_OK;
 }

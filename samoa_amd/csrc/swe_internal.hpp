@@ -94,6 +94,8 @@ struct StepArgs {
     // [n_scen * MEET_SLOTS]: the last workgroup of each scenario publishes
     // the results; no finalize kernel follows.  Null: one does.
     Meet *meet;
+    const uint32_t *lists;                 // [nchunks * list_words(chunk)] the chunks' edge lists, or
+                                           // null: each workgroup builds its own
     // refinement flags from surface-elevation jumps between wet neighbours
     // of the state the step reads (refine above jump_refine, coarsen below
     // jump_coarsen) instead of volume_op's |dQ_h| criterion
@@ -122,6 +124,7 @@ struct AdjArgs {
     const Scen *scen;
     const int32_t *chunk_scen;
     int64_t nchunks;
+    const uint32_t *lists;                  // as in StepArgs
     const double *dt_dev;                   // [n_scen] dt per scenario, or null: use dt
     double dt;
     double g, inv16g;
@@ -234,6 +237,9 @@ constexpr int64_t CHAIN_CHUNKS = 1024;
 // The step of a single mesh whose nbr holds plain neighbour cells
 // (StepArgs::raw_nbr), chunk DEFAULT_CHUNK, one workgroup per chunk, flags
 // by volume_op's criterion; then the finalize kernel.
+// Stores the chunks' edge lists (StepArgs::lists) of the meshes of `a`.
+size_t edge_list_bytes(int64_t nchunks, int chunk);
+hipError_t build_edge_lists(const StepArgs &a, int chunk, uint32_t *lists, hipStream_t s);
 hipError_t launch_step_raw(const StepArgs &a, int solver, hipStream_t s);
 
 }  // namespace swe

@@ -145,12 +145,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
     // CLEAR: 1/h and sqrt(g h) of each cell (clear_cell); TOL: sqrt(g h) (0 when dry)
     __shared__ double s_x[CLEAR ? 2 : 1][CLEAR || TOL ? CH : 1];
     __shared__ double s_f[4][3][CH];  // flux (h, hu, hv, s) per (edge, cell)
-    // The edges to solve: those inside the chunk first, then those leaving it
-    // (to other chunks or the boundary), then the packed neighbours of the
-    // latter.  A chunk of m cells of a validated mesh has at least m - 1
-    // inner edges (consecutive cells share one), so at most m + 2 leave it:
-    // inner + 2 leaving = (3 m + 3 leaving) / 2 <= 3 m + 3 entries.  RAW
-    // meshes are not validated; their neighbours are read again instead.
+    // The edge list (swe_device.hpp).  RAW meshes are not validated: their
+    // leaving edges' neighbours are read again instead of listed.
     __shared__ uint32_t s_list[3 * CH + 4];
     __shared__ uint32_t s_jb[JUMPS ? CH / 16 : 1];  // elevation-jump bits, 2 per cell
     __shared__ int s_wsum[NW];
@@ -212,6 +208,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
         const int32_t *const c_nbr = a.nbr + 3 * (gt + lbase);
         const int8_t *const c_plot = a.plotter + gt + lbase;
         const int8_t *const c_depth = a.depth + gt + lbase;
+        const uint32_t *const list =
+            !RAW && a.lists ? a.lists + (uint64_t)chunk * list_words(CH) : nullptr;
         const int64_t c_out = gs + lbase;  // first output cell of the chunk
         double dt = a.device_dt ? scalar(a.slots)[s].dt
                                 : (a.dt_host ? scalar(a.dt_host)[s] : a.dt);
@@ -226,16 +224,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
             for (int i0 = t; i0 < n; i0 += NT) fastest = max_f64(fastest, pm[i0]);
         }
 
+        // the stored list, or this thread's cell's neighbours to build it from
         int32_t nb[3] = {-1, -1, -1};
         int plot = 1;
-        double my_e = 0.0, my_u = 0.0, my_v = 0.0;  // TOL: this thread's cell state
-        if (active) {
-            // every load goes out before the arithmetic that waits for the state
-            const double e = c_eta[t], u = c_hu[t], vv = c_hv[t], bb = c_b[t];
+        uint32_t head = 0;
+        ListAhead<CH, NT> ahead;
+        if (list) {
+            head = scalar(list)[0];
+            ahead.load(list, t);
+        } else if (active) {
             nb[0] = c_nbr[3 * t];
             nb[1] = c_nbr[3 * t + 1];
             nb[2] = c_nbr[3 * t + 2];
             plot = c_plot[t];
+        }
+        double my_e = 0.0, my_u = 0.0, my_v = 0.0;  // TOL: this thread's cell state
+        if (active) {
+            // every load goes out before the arithmetic that waits for the state
+            const double e = c_eta[t], u = c_hu[t], vv = c_hv[t], bb = c_b[t];
             if constexpr (TOL) {
                 my_e = e;
                 my_u = u;
@@ -272,34 +278,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
         }
         if (JUMPS && t < CH / 16) s_jb[t] = 0;
 
-        // Edges this thread's cell must solve: those leaving the chunk, and
-        // the inner ones whose other cell the traversal visits later.  Inner
-        // edges are so solved from their left side.
-        int inner = 0, leave = 0;
-        if (active) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int32_t p = nb[k];
-                const int lo = (RAW ? p : p >> 2) - lbase;  // chunk-local neighbour
-                const bool inside = p >= 0 && (uint32_t)lo < (uint32_t)cnt;
-                if (!inside) leave |= 1 << k;
-                else if (a.forward ? lo > t : lo < t) inner |= 1 << k;
-            }
-        }
-        // workgroup exclusive prefixes of both counts (0..3 each) via ballots,
-        // packed: inner in the low half, leaving in the high half
-        const int nin = __popc(inner), nout = __popc(leave);
-        const uint64_t i0 = __ballot(nin & 1), i1 = __ballot(nin & 2);
-        const uint64_t o0 = __ballot(nout & 1), o1 = __ballot(nout & 2);
-        const int wpre = lanes_below(i0) + 2 * lanes_below(i1) +
-                         ((lanes_below(o0) + 2 * lanes_below(o1)) << 16);
-        if (lane == 0)
-            s_wsum[wave] = __popcll(i0) + 2 * __popcll(i1) +
-                           ((__popcll(o0) + 2 * __popcll(o1)) << 16);
         if (!RAW && a.prev_max) {
             const double w = wave_max(fastest);
             if (lane == 63) s_wmax[wave] = w;
         }
+        int2 entries;
+        if (list) {
+            entries = ahead.put(list, head, t, s_list);
+        } else {
+            // a plain neighbour's edge back to this cell (two cells of a
+            // conforming mesh share at most one edge)
+            auto back = [&](int k, int lo) -> int {
+                if (!RAW) return nb[k] & 3;
+                return s_nbr[lo] == lbase + t ? 0 : (s_nbr[CH + lo] == lbase + t ? 1 : 2);
+            };
+            auto put = [&](int i, uint32_t ent) { s_list[i] = ent; };
+            entries = list_edges<NT, RAW>(t, cnt, lbase, nb, plot, s_wsum, back, put);
+        }
+        const int n_inner = entries.x, total = entries.y;
         __syncthreads();
         if (!RAW && a.prev_max && t == 0) {
             double m = s_wmax[0];
@@ -307,38 +303,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
             for (int w = 1; w < NW; ++w) m = max_f64(m, s_wmax[w]);
             s_dt = next_dt(sc.courant, sc.dt_clamp, cfl_minimum(sc.scaling, m));
         }
-        int pre = wpre, sum = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const int ws = s_wsum[w];
-            pre += w < wave ? ws : 0;
-            sum += ws;
-        }
-        const int n_inner = sum & 0xffff, total = n_inner + (sum >> 16);
-        int pi = pre & 0xffff, po = n_inner + (pre >> 16);
-        // outward normal of edge k: plotter type p > 0 turns the normals at
-        // 180 + 45 p, 45 + 45 p and 270 + 45 p degrees, p < 0 mirrors the legs
-        const int turn = plot < 0 ? -plot : plot;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int d0 = k == 1 ? 1 : ((k == 0) == (plot > 0) ? 4 : 6);
-            const int32_t p = nb[k];
-            const bool in = inner & (1 << k), out = leave & (1 << k);
-            const int lo = (RAW ? p : p >> 2) - lbase;
-            int ko = p & 3;
-            // a plain neighbour's edge back to this cell (two cells of a
-            // conforming mesh share at most one edge)
-            if (RAW && in) ko = s_nbr[lo] == lbase + t ? 0 : (s_nbr[CH + lo] == lbase + t ? 1 : 2);
-            const uint32_t other = in ? ((uint32_t)lo << 11) | ((uint32_t)ko << 20)
-                                      : LEAVES | (p < 0 ? BOUNDARY : 0u);
-            if (in || out)
-                s_list[in ? pi : po] = (uint32_t)t | ((uint32_t)k << 9) |
-                                       ((uint32_t)((turn + d0) & 7) << 22) | other;
-            if (!RAW && out) s_list[po + total - n_inner] = (uint32_t)p;
-            pi += in ? 1 : 0;
-            po += out ? 1 : 0;
-        }
-        __syncthreads();
+        // inner edges are solved from their left side: the lower cell when
+        // forward, the upper when backward, whose normal is the opposite one
+        const int left = a.forward ? 0 : 11, right = 11 - left;
+        const uint32_t opposite = a.forward ? 0u : 4u;
 
         __builtin_amdgcn_s_setprio(0);
         // One pass over the list.  FIRST: a GeoClaw kernel's pass with clear_flux,
@@ -353,7 +321,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
         for (int e = t; e < total; e += NT, bit <<= 1) {
             if (!FIRST && !(rounds & bit)) continue;
             const uint32_t ent = s_list[e];
-            const int lc = ent & 511, k = (ent >> 9) & 3, dir = (ent >> 22) & 7;
+            const bool inside = !(ent & LEAVES);
+            const int lc = (ent >> left) & 511, k = (ent >> (left + 9)) & 3;
+            const uint32_t dir = ((ent >> 22) & 7) ^ (inside ? opposite : 0u);
             double nx = s_dir[dir][0], ny = s_dir[dir][1];
             // the two cells' quantities: left and right for an inner edge;
             // one that leaves the chunk may need them exchanged
@@ -362,8 +332,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
             for (int m = 0; m < 4; ++m) L[m] = s_q[m][lc];
             if (SHORT || TOL) L[4] = s_x[0][lc];
             if (SHORT && CLEAR) L[5] = s_x[CLEAR ? 1 : 0][lc];
-            const bool inside = !(ent & LEAVES);
-            const int lo = (ent >> 11) & 511;
+            const int lo = (ent >> right) & 511;
             bool flip = false;
             uint32_t jb = 0;
             if (inside) {
@@ -467,7 +436,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
             s_f[2][k][lc] = fL.hv;
             s_f[3][k][lc] = fL.s;
             if (inside) {
-                const int ko = (ent >> 20) & 3;
+                const int ko = (ent >> (right + 9)) & 3;
                 s_f[0][ko][lo] = fR.h;
                 s_f[1][ko][lo] = fR.hu;
                 s_f[2][ko][lo] = fR.hv;
@@ -687,6 +656,47 @@ hipError_t upload_tables(const double *normal, const double *leg) {
 
 hipError_t launch_finalize(const StepArgs &a, hipStream_t s) {
     hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)a.n_scen), dim3(FIN_THREADS), 0, s, a);
+    return hipGetLastError();
+}
+
+// The edge list of each chunk: the step kernels' own (list_edges), stored.
+template <int CH>
+__global__ __launch_bounds__(CH) void edge_list_kernel(StepArgs a, uint32_t *lists) {
+    __shared__ int s_wsum[CH / 64];
+    const int t = threadIdx.x;
+    const uint32_t chunk = blockIdx.x;
+    const int s = a.chunk_scen ? a.chunk_scen[chunk] : 0;
+    const Scen sc = a.chunk_scen ? a.scen[s] : a.scen0;
+    const int32_t lbase = (int32_t)(chunk - (uint32_t)sc.chunk_off) * CH;
+    const int cnt = (int)((sc.n - lbase) < CH ? (sc.n - lbase) : CH);
+    const int32_t *const nbr = a.nbr + 3 * (sc.topo_off + lbase);
+    int32_t nb[3] = {-1, -1, -1};
+    int plot = 1;
+    if (t < cnt) {
+        nb[0] = nbr[3 * t];
+        nb[1] = nbr[3 * t + 1];
+        nb[2] = nbr[3 * t + 2];
+        plot = a.plotter[sc.topo_off + lbase + t];
+    }
+    uint32_t *const list = lists + (uint64_t)chunk * list_words(CH);
+    const int2 n = list_edges<CH, false>(
+        t, cnt, lbase, nb, plot, s_wsum, [&](int k, int) { return nb[k] & 3; },
+        [&](int i, uint32_t ent) { list[LIST_HEAD + i] = ent; });
+    if (t == 0) list[0] = (uint32_t)n.x | ((uint32_t)n.y << 16);
+}
+
+size_t edge_list_bytes(int64_t nchunks, int chunk) {
+    return sizeof(uint32_t) * (size_t)list_words(chunk) * (size_t)nchunks;
+}
+
+hipError_t build_edge_lists(const StepArgs &a, int chunk, uint32_t *lists, hipStream_t s) {
+    const dim3 grid((unsigned)a.nchunks);
+    switch (chunk) {
+        case 128: edge_list_kernel<128><<<grid, 128, 0, s>>>(a, lists); break;
+        case 256: edge_list_kernel<256><<<grid, 256, 0, s>>>(a, lists); break;
+        case 512: edge_list_kernel<512><<<grid, 512, 0, s>>>(a, lists); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

@@ -240,6 +240,10 @@ void stage_give(int k, char *p) {
 // Traversals of a changed mesh after which its edge lists are stored.
 constexpr int64_t LISTS_FROM = 2;
 
+// Steps of a run on a caller's stream from which they form a chain: it saves
+// about 1 us a step against workgroups that meet, its end costs 4 us.
+constexpr int64_t CHAIN_LEAST = 6;
+
 struct Batch {
     int device = 0;
     hipStream_t stream = nullptr;      // where work is launched (caller may replace it)
@@ -905,11 +909,19 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
                                hipMemcpyHostToDevice, B.stream));
     }
 
-    SWE_TRY(lists_for(B, n_steps));
+    // A caller may capture single steps on a stream of its own and replay them:
+    // nothing is prepared or waited for there, every step takes its dt from the
+    // slots and leaves the next one in them.
+    const bool own = B.stream == B.own_stream;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (!own) HIP_TRY(hipStreamIsCapturing(B.stream, &capture));
+    const bool captured = capture != hipStreamCaptureStatusNone;
+    if (!captured) SWE_TRY(lists_for(B, n_steps));
     // Meshes of few chunks step in a chain: a step forms its dt from the
     // partials of the one before, and a finalize kernel runs only for who
-    // reads the results.
-    bool chain = true;
+    // reads the results.  On a caller's stream the chain ends with the call (so
+    // that a capture finds the slots current), which a short one isn't worth.
+    bool chain = own || (!captured && n_steps >= CHAIN_LEAST);
     for (auto &s : B.scen) chain = chain && s.nchunks <= swe::CHAIN_CHUNKS;
     if (!chain) SWE_TRY(chain_flush(B));
     // one step from state buffer `from`; in a chain, with the partials
@@ -989,8 +1001,8 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     }
     if (left > 0) SWE_TRY(single());
     if (n_steps > 0) B.flags_valid = B.keep_flags != 0;
+    if (!own || time || dt_next) SWE_TRY(chain_flush(B));
     if (!time && !dt_next) return SWE_OK;
-    SWE_TRY(chain_flush(B));
     std::vector<swe::Slots> res((size_t)B.nscen);
     const Part part{B.d_slots, res.data(), sizeof(swe::Slots) * res.size()};
     SWE_TRY(transfer(B, &part, 1, true));
@@ -1364,6 +1376,7 @@ int batch_adjoint_device(Batch &B, const double *eta, const double *hu, const do
 }
 
 int batch_set_stream(Batch &B, void *stream) {
+    SWE_TRY(chain_flush(B));
     HIP_TRY(hipStreamSynchronize(B.stream));
     B.stream = stream ? (hipStream_t)stream : B.own_stream;
     return SWE_OK;

@@ -12,10 +12,10 @@ namespace swe {
 constexpr int CHUNK_SIZES[3] = {128, 256, 512};
 constexpr int DEFAULT_CHUNK = 256;
 
-// Per-scenario results and device dt chain.  The finalize kernel that follows
-// a step kernel on the stream writes them; the step kernel reads dt.  Steps
-// in a chain (StepArgs::chained) run without a finalize kernel between them:
-// each advances time, and the one after it forms its dt from the partials.
+// Per-scenario results and device dt chain, read by the step kernel and written
+// by the finalize kernel that follows it, or by the last of its workgroups
+// (StepArgs::meet).  Steps in a chain (StepArgs::chained) do neither between
+// them: each advances time, and the one after it forms its dt from the partials.
 struct Slots {
     double dt;                   // dt of the next step (device dt chain)
     double time;                 // simulated time (device dt chain)
@@ -234,12 +234,12 @@ hipError_t launch_finalize(const StepArgs &a, hipStream_t s);
 // reads from L2.  100 steps: 1.33 -> 1.06 ms at 128 chunks, 2.81 -> 2.39 at
 // 1024; at 2048, 4.24 -> 4.15, and 4.05 where the workgroups meet instead.
 constexpr int64_t CHAIN_CHUNKS = 1024;
-// The step of a single mesh whose nbr holds plain neighbour cells
-// (StepArgs::raw_nbr), chunk DEFAULT_CHUNK, one workgroup per chunk, flags
-// by volume_op's criterion; then the finalize kernel.
 // Stores the chunks' edge lists (StepArgs::lists) of the meshes of `a`.
 size_t edge_list_bytes(int64_t nchunks, int chunk);
 hipError_t build_edge_lists(const StepArgs &a, int chunk, uint32_t *lists, hipStream_t s);
+// The step of a single mesh whose nbr holds plain neighbour cells
+// (StepArgs::raw_nbr), chunk DEFAULT_CHUNK, one workgroup per chunk, flags
+// by volume_op's criterion; then the finalize kernel.
 hipError_t launch_step_raw(const StepArgs &a, int solver, hipStream_t s);
 
 }  // namespace swe

@@ -4,17 +4,17 @@
 // every mesh of a batch: the GeoClaw flux on every edge (skeleton_scalar_op
 // :196-215 and bnd_skeleton_scalar_op :231-255), the cell update with the
 // wet/dry limiter (cell_update_op :257-284, volume_op :307-355) and each
-// chunk's CFL / refinement partials.  A small finalize kernel then reduces
-// the partials per scenario and advances the dt chain
-// (post_traversal_grid_op :111-131, pre_traversal_grid_op :89-109).  The step
-// kernel uses no atomics: per-workgroup atomics on one per-scenario address
-// serialise across the eight XCDs.
+// chunk's CFL / refinement partials.  The partials of a scenario are reduced,
+// and the dt chain advanced (post_traversal_grid_op :111-131,
+// pre_traversal_grid_op :89-109), in one of three ways: by the next step of a
+// chain of them (CHAIN_CHUNKS), by the last workgroup to meet the others
+// (MEET_CHUNKS), or by a small finalize kernel.
 //
 // Mapping.  A workgroup processes chunks of CH consecutive SFC cells of one
-// scenario (one thread per cell).  It stages the chunk's state in LDS, builds
-// a compact list of the edges it must solve (each edge inside the chunk once,
-// from its left side; edges to cells outside the chunk and domain-boundary
-// edges by this chunk), solves them with one thread per list entry, scatters
+// scenario.  It stages the chunk's state in LDS with a compact list of the edges
+// it must solve (each edge inside the chunk once, from its left side; edges to
+// cells outside the chunk and domain-boundary edges by this chunk), which is
+// stored with the mesh or built here, solves them with one thread per list entry, scatters
 // both sides' fluxes into LDS, then updates its cells and reduces the CFL
 // candidate.  The Sierpinski order keeps almost every neighbour inside the
 // chunk, so ~1.6 Riemann solves per cell are done instead of 3, and halo
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
         }
 
         // CFL minimum and refinement count of the chunk (post_traversal_grid_op
-        // :117-118); the finalize kernel reduces the chunks of each scenario.
+        // :117-118), reduced over the scenario here, later, or in the next step.
         const double wmax = wave_max(speed);
         const int wref = __popcll(__ballot(refined));
         if (lane == 63) {

@@ -224,3 +224,39 @@ def test_cells_without_numbers_set_no_limit():
         op.upload(*bad)
         assert op.run(3, 1e-3, True)[1] == COURANT * huge
     op.close()
+
+
+@pytest.mark.parametrize("depth", [10, 18, 20])  # meeting workgroups, and a finalize kernel
+def test_captured_steps_replay(depth):
+    """Two single steps captured on the caller's stream: every replay goes on
+    with the dt chain, also between the handle's own runs."""
+    import torch
+
+    print("case:", depth, flush=True)
+    mesh = host.mesh_uniform(depth)
+    st = beach(mesh, 3)
+    dt0 = host.initial_dt(mesh, st, COURANT) * 1e3
+    ref = HostChain(mesh, st, dt0)
+    op = operator(mesh)
+    op.upload(*st)
+    op.run(1, dt0, False)
+    op.run(2, None, True, wait=False)  # a chain on the handle's own stream
+    stream = torch.cuda.Stream()
+    op.set_stream(stream.cuda_stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        op.run(1, None, True, wait=False)
+        op.run(1, None, False, wait=False)
+    ref.run(3)
+    for k in range(3):
+        with torch.cuda.stream(stream):
+            graph.replay()
+        ref.run(2)
+        n = (0, 8, 2)[k]
+        op.run(n, None, True, wait=False)
+        ref.run(n)
+        assert op.run(0, None, True) == (ref.t, ref.dt)
+        for a, b in zip(op.download(), ref.op.download()):
+            assert np.array_equal(a, b)
+    op.close()
+    ref.op.close()

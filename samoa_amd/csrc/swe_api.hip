@@ -127,8 +127,8 @@ int ensure_tables(int device) {
     return SWE_OK;
 }
 
-// The captured pair of steps bakes in which buffer holds the state, the
-// starting direction and the launch shape; a pair returns the state to the
+// The captured steps bake in which buffer holds the state, the starting
+// direction and the launch shape; an even number of them returns the state to the
 // buffer it started from, so the graph stays valid across run calls.  A
 // handle keeps one per (state buffer, starting direction): a run of an odd
 // number of steps leaves the next run in the other buffer or direction, which
@@ -239,6 +239,16 @@ void stage_give(int k, char *p) {
 
 // Traversals of a changed mesh after which its edge lists are stored.
 constexpr int64_t LISTS_FROM = 2;
+
+// Steps of a captured graph (an even number: the state's buffers, the direction
+// and the partials are then where they were), and of a run that is worth it.  A
+// graph launch costs the device 3-4 us, a launch from the host 0.4 us more than
+// the same kernel in a graph: 100 steps of 128 chunks 919 us in graphs of two,
+// 731 one by one, 733 in graphs of 8, 693 of 24; of 2048 chunks, toleranced, with
+// the download, 2990, 2715, 2715, 2650.  Capturing takes 70 us (100 steps with the
+// capture 1160 us in twos, 905 one by one, 970 in graphs of 24).
+constexpr int GRAPH_STEPS = 24;
+constexpr int64_t GRAPH_FROM = 2 * GRAPH_STEPS;
 
 // Steps of a run on a caller's stream from which they form a chain: it saves
 // about 1 us a step against workgroups that meet, its end costs 4 us.
@@ -958,8 +968,7 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     // the first step of a chain, and the first after a remeshing, reads its
     // dt from elsewhere than the captured ones
     if (chain && left > 0 && (!B.pending || B.pend_chunks != B.nchunks)) SWE_TRY(single());
-    const int64_t pairs = left / 2;
-    if (pairs > 0) {
+    if (left >= GRAPH_FROM) {
         GraphCache &gc = B.graph[B.cur][fwd];
         const int pp = chain ? B.pp : -1;
         if (!gc.exec || gc.cur != B.cur || gc.forward != fwd || gc.chunk != B.chunk ||
@@ -974,16 +983,16 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
             HIP_TRY(hipStreamSynchronize(B.stream));
             hipGraph_t graph;
             HIP_TRY(hipStreamBeginCapture(B.own_stream, hipStreamCaptureModeThreadLocal));
-            hipError_t e1 = one_step(B.own_stream, B.cur, fwd, true, B.pp);
-            hipError_t e2 =
-                e1 == hipSuccess ? one_step(B.own_stream, 1 - B.cur, 1 - fwd, true, 1 - B.pp) : e1;
-            hipError_t e3 = hipStreamEndCapture(B.own_stream, &graph);
-            if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess)
+            hipError_t e1 = hipSuccess;
+            for (int i = 0; i < GRAPH_STEPS && e1 == hipSuccess; ++i)
+                e1 = one_step(B.own_stream, B.cur ^ (i & 1), fwd ^ (i & 1), true, B.pp ^ (i & 1));
+            const hipError_t e2 = hipStreamEndCapture(B.own_stream, &graph);
+            if (e1 != hipSuccess || e2 != hipSuccess)
                 return fail(SWE_ERR_HIP, "run: graph capture failed: %s",
-                            hipGetErrorString(e1 != hipSuccess ? e1 : (e2 != hipSuccess ? e2 : e3)));
-            hipError_t e4 = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
+                            hipGetErrorString(e1 != hipSuccess ? e1 : e2));
+            const hipError_t e3 = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
             (void)hipGraphDestroy(graph);
-            if (e4 != hipSuccess) return fail(SWE_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e4));
+            if (e3 != hipSuccess) return fail(SWE_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e3));
             gc.cur = B.cur;
             gc.forward = fwd;
             gc.chunk = B.chunk;
@@ -996,10 +1005,10 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
             gc.jump_refine = B.jump_refine;
             gc.jump_coarsen = B.jump_coarsen;
         }
-        for (int64_t i = 0; i < pairs; ++i) HIP_TRY(hipGraphLaunch(gc.exec, B.stream));
-        left -= 2 * pairs;
+        for (; left >= GRAPH_STEPS; left -= GRAPH_STEPS)
+            HIP_TRY(hipGraphLaunch(gc.exec, B.stream));
     }
-    if (left > 0) SWE_TRY(single());
+    while (left > 0) SWE_TRY(single());
     if (n_steps > 0) B.flags_valid = B.keep_flags != 0;
     if (!own || time || dt_next) SWE_TRY(chain_flush(B));
     if (!time && !dt_next) return SWE_OK;

@@ -260,3 +260,26 @@ def test_captured_steps_replay(depth):
             assert np.array_equal(a, b)
     op.close()
     ref.op.close()
+
+
+# around the length from which steps go into a graph (48, and 24 in each), from
+# either buffer and direction
+@pytest.mark.parametrize("depth", [6, 18, 19])
+def test_long_runs_equal_single_traversals(depth):
+    print("case:", depth, flush=True)
+    mesh = host.mesh_uniform(depth)
+    st = beach(mesh, 4)
+    dt0 = host.initial_dt(mesh, st, COURANT) * 1e3
+    ref = HostChain(mesh, st, dt0)
+    op = operator(mesh, 128 if depth == 19 else None)
+    op.upload(*st)
+    fwd = False
+    for i, n in enumerate([48, 49, 47, 74, 121]):
+        got = op.run(n, dt0 if i == 0 else None, fwd)
+        ref.run(n)
+        fwd ^= n % 2 == 1
+        assert got == (ref.t, ref.dt)
+        for a, b in zip(op.download(), ref.op.download()):
+            assert np.array_equal(a, b)
+    op.close()
+    ref.op.close()

@@ -33,6 +33,7 @@
 // at corner (k+1) mod 3, half 1 the half at corner (k+2) mod 3.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 
 #include "swe_internal.hpp"
@@ -42,11 +43,10 @@ namespace swe {
 namespace {
 
 constexpr int AT = 256;           // threads per workgroup of the per-cell kernels
-// the emit kernels' workgroups, measured: the kept-cell emit streams over
-// every cell (larger workgroups, fewer of them), the changing-cell emit and
-// link run over the ~5 % that change (smaller ones, spread over more CUs)
-constexpr int KEEP_T = 512;
-constexpr int CHANGE_T = 128;
+// threads per workgroup of the emit and the link: the ~5 % of cells that change
+// spread over more CUs in small ones, and for the kept cells 512 are no faster
+// (84.0 against 84.5 us at 4.6 M cells)
+constexpr int EMIT_T = 128;
 constexpr int SCAN_T = 256;       // scan: threads per tile
 constexpr int SCAN_ITEMS = 8;     // scan: consecutive items per thread
 constexpr int SCAN_TILE = SCAN_T * SCAN_ITEMS;
@@ -706,7 +706,7 @@ __device__ double raster_wave(const AdaptArgs &a, const double c[6], int levels)
     return v;
 }
 
-// A new cell of more halvings than this leaves its b to raster_kernel: a
+// A new cell of more halvings than this leaves its b to raster_children: a
 // child at depth 11 of a depth-18 run averages 1024 samples, a serial chain of
 // gathers that held one thread, and the emit with it, for 3.1-3.8 ms of every
 // changing remeshing; a wave per child takes 6-15 us.  Two samples at most
@@ -730,8 +730,7 @@ __device__ __forceinline__ void put_slot(int32_t *eslot, int64_t c, int k, int h
 // its pairing from link_kernel, which writes both sides of every edge of the
 // changing cells.  Writing all three entries makes the neighbour store one
 // 12-B store per lane, dense across the wave.
-__global__ __launch_bounds__(KEEP_T) void emit_keep_kernel(AdaptArgs a) {
-    const int64_t c = blockIdx.x * (int64_t)KEEP_T + threadIdx.x;
+__device__ __forceinline__ void emit_keep(const AdaptArgs &a, int64_t c) {
     if (c >= a.n) return;
     if (c == 0 && a.scen_dev) *a.scen_dev = a.scen_new;  // no host upload of the table
     // every load, the neighbours' new indices included, is issued before the
@@ -747,7 +746,7 @@ __global__ __launch_bounds__(KEEP_T) void emit_keep_kernel(AdaptArgs a) {
                   k2 = a.kidx[q2 >= 0 ? q2 >> 2 : c];
     asm volatile("" ::"v"((int)dc), "v"((int)pc), "v"(oc), "v"(ec), "v"(uc), "v"(vc), "v"(bc), "v"(k0),
                  "v"(k1), "v"(k2));
-    if (kc < 0) return;  // a changing cell: emit_change_kernel
+    if (kc < 0) return;  // a changing cell: emit_change
     const int64_t b0 = kc;
     a.depth_out[b0] = dc;
     a.plotter_out[b0] = pc;
@@ -768,8 +767,7 @@ __global__ __launch_bounds__(KEEP_T) void emit_keep_kernel(AdaptArgs a) {
 // children's types; the grandchildren's types.  The state stays in registers: as far as the
 // compiler knows, the new cells' stores could alias the old arrays, and it
 // would read them again after every store.
-__global__ __launch_bounds__(CHANGE_T) void emit_change_kernel(AdaptArgs a) {
-    const int64_t i = blockIdx.x * (int64_t)CHANGE_T + threadIdx.x;
+__device__ __forceinline__ void emit_change(const AdaptArgs &a, int64_t i) {
     if (i >= a.n_changing) return;
     const int64_t c = a.list[i];
     const int64_t c1 = c + 1 < a.n ? c + 1 : c;
@@ -853,20 +851,37 @@ __global__ __launch_bounds__(CHANGE_T) void emit_change_kernel(AdaptArgs a) {
     }
 }
 
-// b of the children that emit_change_kernel left (raster_list: their split
-// cells, in any order): a workgroup per split cell, a wave per child.
-constexpr int RASTER_T = 256, RASTER_BLOCKS = 2048;
-__global__ __launch_bounds__(RASTER_T) void raster_kernel(AdaptArgs a) {
+// The new mesh: the changing cells in the first change_blocks workgroups, the
+// kept ones in the others.  A kept cell moves 112 B, which bounds the launch on a
+// large mesh (84 us at 4.6 M cells, 6.1 TB/s); a changing one is a chain of four
+// loads, which bounds it on a small one.  In two launches, kept cells with 512
+// threads, the changing ones waited behind the others: 84.5 + 10.8 us; 50 steps
+// with remeshing 2.72 -> 2.51 ms at 35 k cells, 3.46 -> 3.25 at 139 k, 7.63 ->
+// 7.30 at 1.27 M, 100 steps at 4.6 M 48.3 -> 47.4.
+__global__ __launch_bounds__(EMIT_T) void emit_kernel(AdaptArgs a, unsigned change_blocks) {
+    if (blockIdx.x < change_blocks)
+        emit_change(a, blockIdx.x * (int64_t)EMIT_T + threadIdx.x);
+    else
+        emit_keep(a, (blockIdx.x - change_blocks) * (int64_t)EMIT_T + threadIdx.x);
+}
+
+// b of the children that emit_change left (raster_list: their split cells, in
+// any order), by this wave and those of the other blocks: each takes one child
+// at a time.
+constexpr unsigned RASTER_BLOCKS = 4096;
+__device__ __forceinline__ void raster_children(const AdaptArgs &a, unsigned blocks) {
+    constexpr unsigned W = EMIT_T / 64;
     const uint32_t count = *a.raster_count;
-    const int j = threadIdx.x >> 6;  // the child
-    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-        const int64_t c = a.raster_list[i];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(blockIdx.x * W + threadIdx.x / 64);
+    for (uint64_t k = wave; k < 4 * (uint64_t)count; k += blocks * W) {
+        const int64_t c = a.raster_list[k / 4];
+        const int j = (int)(k % 4);
         const int pat = a.code[c] - CODE_SPLIT;
         if (j >= 2 + (pat & 1) + (pat >> 1)) continue;
         const int64_t idx = (a.base[c] & 0xffffffffLL) + j;
         const int dc = a.depth_out[idx];
         const int levels = raster_levels(a, dc);
-        if (levels <= RASTER_INLINE) continue;  // written by emit_change_kernel
+        if (levels <= RASTER_INLINE) continue;  // written by emit_change
         double q[6];
         tree_corners(a.off_out[idx], 0, dc, q);
         const double v = raster_wave(a, q, levels);
@@ -881,8 +896,13 @@ __global__ __launch_bounds__(RASTER_T) void raster_kernel(AdaptArgs a) {
 // type; the neighbours' types and new indices; the slots of the neighbours
 // that change (read at every lane, at an index in range, and used where the
 // neighbour changes).
-__global__ __launch_bounds__(CHANGE_T) void link_kernel(AdaptArgs a) {
-    const int64_t i = blockIdx.x * (int64_t)CHANGE_T + threadIdx.x;
+// The first raster_blocks workgroups sample b for the split cells instead: their
+// chains of gathers are the longest, and a launch of their own took 4.7 us with
+// nothing to sample, 13 with the gap before it on a small mesh (50 steps with
+// remeshing: 2.87 -> 2.70 ms at 35 k cells, 3.63 -> 3.46 at 139 k).
+__global__ __launch_bounds__(EMIT_T) void link_kernel(AdaptArgs a, unsigned raster_blocks) {
+    if (blockIdx.x < raster_blocks) return raster_children(a, raster_blocks);
+    const int64_t i = (blockIdx.x - raster_blocks) * (int64_t)EMIT_T + threadIdx.x;
     if (i >= a.n_changing) return;
     const int64_t c = a.list[i];
     const int pc = a.plotter[c];
@@ -1155,14 +1175,14 @@ hipError_t adapt_emit(const AdaptArgs &args, hipStream_t s, bool prefix_done) {
     if (tiles > 0 && !prefix_done)
         scan_codes_kernel<<<(unsigned)tiles, SCAN_T, 0, s>>>(a.n, a.code, a.bsum, a.base, a.kidx,
                                                              a.list);
-    emit_keep_kernel<<<blocks_for(a.n, KEEP_T), KEEP_T, 0, s>>>(a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.n_changing == 0) return e;
-    emit_change_kernel<<<blocks_for(a.n_changing, CHANGE_T), CHANGE_T, 0, s>>>(a);
-    link_kernel<<<blocks_for(a.n_changing, CHANGE_T), CHANGE_T, 0, s>>>(a);
-    if (a.raster_list)
-        raster_kernel<<<(unsigned)(a.n_changing < RASTER_BLOCKS ? a.n_changing : RASTER_BLOCKS),
-                        RASTER_T, 0, s>>>(a);
+    const unsigned changing = blocks_for(a.n_changing, EMIT_T);
+    emit_kernel<<<changing + blocks_for(a.n, EMIT_T), EMIT_T, 0, s>>>(a, changing);
+    if (changing > 0) {
+        const int64_t waves = 4 * a.n_changing;  // at most
+        const unsigned raster =
+            !a.raster_list ? 0 : (unsigned)std::min<int64_t>(waves * 64 / EMIT_T, RASTER_BLOCKS);
+        link_kernel<<<raster + changing, EMIT_T, 0, s>>>(a, raster);
+    }
     return hipGetLastError();
 }
 

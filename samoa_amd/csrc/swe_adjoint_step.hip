@@ -27,7 +27,7 @@
 // fifth of it dry) from 61 to 35 us.  The general pass alone needs 206
 // registers: held to 168 it spills 76 bytes on its few edges, and three waves
 // per SIMD instead of two hide more of the first pass's LDS and memory waits:
-// 213.7 us at the start, 122 with two waves, 106 with three.  LDS (50 KB for
+// 213.7 us with neither, 122 with two waves, 106 with three.  LDS (50 KB for
 // 256 cells) allows no fourth.  The f-wave kernel went from 107 to 81 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -45,9 +45,10 @@ namespace swe {
 __constant__ double c_normal_adj[17 * 3 * 2];  // [plotter + 8][edge][x,y]
 __constant__ double c_leg_adj[64];             // l(k) = sqrt(0.5)**k at k + 1
 
-// (the LDS of 512 cells allows two waves per SIMD)
-template <int SOLVER, int CH>
-__global__ __launch_bounds__(CH) __attribute__((amdgpu_waves_per_eu(CH == 512 ? 2 : 3))) void
+// NT threads work on a chunk, CH or 2 CH; the first CH hold a cell each.  512 of
+// them fill two waves per SIMD, as does the LDS of 512 cells.
+template <int SOLVER, int CH, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 ? 2 : 3))) void
 adjoint_step_kernel(AdjArgs args) {
     __shared__ double s_q[4][CH];     // eta, hu, hv, b of the chunk at t_n
     __shared__ double s_x[2][CH];     // 1/h and sqrt(g h) of each cell (clear_cell)
@@ -57,13 +58,13 @@ adjoint_step_kernel(AdjArgs args) {
     __shared__ uint32_t s_list[3 * CH + 4];  // the edge list (swe_device.hpp)
     __shared__ uint16_t s_rest[3 * CH];  // entries left to the general solver
     __shared__ int8_t s_dep[CH], s_mask[CH];
-    __shared__ int s_wsum[CH / 64], s_nrest;
+    __shared__ int s_wsum[NT / 64], s_nrest;
     __shared__ double s_dir[8][2];  // the unit vectors at multiples of 45 degrees
     __shared__ double s_leg[64];
 
     int t = threadIdx.x;
     if (t < 16) s_dir[t >> 1][t & 1] = c_normal_adj[((((t >> 1) - 2) & 7) + 9) * 6 + 2 + (t & 1)];
-    for (int i = t; i < 64; i += CH) s_leg[i] = c_leg_adj[i];
+    for (int i = t; i < 64; i += NT) s_leg[i] = c_leg_adj[i];
     const uint32_t nchunks = (uint32_t)args.nchunks, q = nchunks / 8, r = nchunks % 8;
     const uint32_t nvirt = 8 * ((nchunks + 7) / 8);
     for (uint32_t v = blockIdx.x; v < nvirt; v += gridDim.x) {
@@ -97,7 +98,7 @@ adjoint_step_kernel(AdjArgs args) {
         int32_t nb[3] = {-1, -1, -1};
         int plot = 1;
         uint32_t head = 0;
-        ListAhead<CH, CH> ahead;
+        ListAhead<CH, NT> ahead;
         if (list) {
             head = scalar(list)[0];
             ahead.load(list, t);
@@ -140,7 +141,7 @@ adjoint_step_kernel(AdjArgs args) {
 
         const int2 entries =
             list ? ahead.put(list, head, t, s_list)
-                 : list_edges<CH, false>(
+                 : list_edges<NT, false>(
                        t, cnt, lbase, nb, plot, s_wsum, [&](int k, int) { return nb[k] & 3; },
                        [&](int i, uint32_t ent) { s_list[i] = ent; });
         const int n_inner = entries.x, total = entries.y;
@@ -161,7 +162,7 @@ adjoint_step_kernel(AdjArgs args) {
         asm volatile("" : "+v"(t), "+s"(ap));
         const auto &a = *ap;
         const double g = a.g;
-        for (int i = t; i < n; i += CH) {
+        for (int i = t; i < n; i += NT) {
             const int e = FIRST ? i : s_rest[i];
             const uint32_t ent = s_list[e];
             const bool inside = !(ent & LEAVES);
@@ -339,8 +340,19 @@ template <int SOLVER, int CH>
 static void launch_adj_t(const AdjArgs &a, int64_t grid_blocks, hipStream_t s) {
     const int64_t nvirt = 8 * ((a.nchunks + 7) / 8);
     const int64_t blocks = grid_blocks > 0 && grid_blocks < nvirt ? grid_blocks : nvirt;
-    hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH>), dim3((unsigned)blocks), dim3(CH), 0, s,
-                       a);
+    // Two threads per cell where every workgroup is resident at once that way (256
+    // CUs of 512 lanes): a chunk's ~1.6 CH edges then take one round, and the
+    // general solver keeps its 205 registers.  A launch, us: 13.8 -> 11.9 at 8
+    // chunks, 15.0 -> 12.8 at 256, with 128-cell chunks 16.9 -> 14.6 at 512, the
+    // f-wave solver 9.0 -> 8.3 at 256; but 17.4 -> 20.9 at 512 chunks, 24.2 -> 31.7
+    // at 1024.
+    constexpr int TWO = CH <= 256 ? 2 * CH : CH;
+    if (CH <= 256 && a.nchunks * TWO <= 256 * 512)
+        hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH, TWO>), dim3((unsigned)blocks),
+                           dim3(TWO), 0, s, a);
+    else
+        hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH, CH>), dim3((unsigned)blocks), dim3(CH),
+                           0, s, a);
 }
 
 hipError_t launch_adjoint(const AdjArgs &a, int solver, int chunk, int64_t grid_blocks,

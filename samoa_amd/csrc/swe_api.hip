@@ -391,15 +391,20 @@ bool all_uploaded(const Batch &B) {
 
 swe::StepArgs make_args(const Batch &B, int from, int to, int forward);
 
-// Brings the device dt of a chain of steps into the slots.
-int chain_flush(Batch &B) {
-    if (!B.pending) return SWE_OK;
+// The finalize kernel's arguments that bring the device dt of a chain of steps into
+// the slots.
+swe::StepArgs flush_args(const Batch &B) {
     swe::StepArgs a = make_args(B, 0, 1, 0);
     a.part_max = B.d_part_max[B.pp];
     a.device_dt = 1;
     a.chained = 1;
     a.prev_chunks = (int32_t)B.pend_chunks;
-    HIP_TRY(swe::launch_finalize(a, B.stream));
+    return a;
+}
+
+int chain_flush(Batch &B) {
+    if (!B.pending) return SWE_OK;
+    HIP_TRY(swe::launch_finalize(flush_args(B), B.stream));
     B.pending = false;
     return SWE_OK;
 }
@@ -934,13 +939,18 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     bool chain = own || (!captured && n_steps >= CHAIN_LEAST);
     for (auto &s : B.scen) chain = chain && s.nchunks <= swe::CHAIN_CHUNKS;
     if (!chain) SWE_TRY(chain_flush(B));
+    // A single step of a larger mesh that nobody waits for leaves its partials too:
+    // a remeshing that follows finalizes them beside a kernel of its own, any
+    // other call before it reads the slots.
+    const bool late = own && !chain && B.nscen == 1 && n_steps == 1 && !time && !dt_next &&
+                      !meet_of(B);
     // one step from state buffer `from`; in a chain, with the partials
     // d_part_max[pp] of the step before if there is one
     auto one_step = [&](hipStream_t st, int from, int fwd, bool prev, int pp) -> hipError_t {
         swe::StepArgs a = make_args(B, from, 1 - from, fwd);
         a.device_dt = 1;
         a.refine = B.keep_flags ? B.refine : nullptr;
-        if (chain) {
+        if (chain || late) {
             a.chained = 1;
             a.skip_finalize = 1;
             a.part_max = B.d_part_max[1 - pp];
@@ -958,7 +968,7 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
         B.cur = 1 - B.cur;
         fwd = 1 - fwd;
         --left;
-        if (chain) {
+        if (chain || late) {
             B.pending = true;
             B.pp = 1 - B.pp;
             B.pend_chunks = B.nchunks;
@@ -1150,8 +1160,12 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
                                B.stream));
     }
     swe::AdaptPlan plan{};
+    const bool late = B.pending && B.pend_chunks > swe::CHAIN_CHUNKS;
+    const swe::StepArgs fin = late ? flush_args(B) : swe::StepArgs{};
     HIP_TRY(swe::adapt_plan(a, B.stream, B.ad_last_sweeps, B.ad_off_valid, B.ad_last_changed,
-                            1 << 16, epoch, B.ad_host, B.ad_host_dev, &B.ad_seq, &plan));
+                            1 << 16, epoch, B.ad_host, B.ad_host_dev, &B.ad_seq,
+                            late ? &fin : nullptr, &plan));
+    if (late) B.pending = false;
     B.ad_last_changed = (plan.status & 2u) != 0;
     const int sweeps = plan.sweeps;
     if (sweeps < 0) return fail(SWE_ERR_STATE, "adapt: the conformity sweeps did not converge");

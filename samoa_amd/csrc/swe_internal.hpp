@@ -193,11 +193,12 @@ struct AdaptPlan {
 // tags their sweep stamps, so that no pass has to clear them).  host: 8
 // words of coherent pinned memory for the results, host_dev its device
 // address; *seq numbers the results (incremented per batch).  Waits for the
-// device once per batch.  adapt_emit then writes the prefix of the counts
-// (base; its high word counts the cells that change) and the new mesh.
+// device once per batch.  late: the finalize kernel's arguments of a step that ran
+// without one (one scenario), or null.  adapt_emit then writes the prefix of the
+// counts (base; its high word counts the cells that change) and the new mesh.
 hipError_t adapt_plan(const AdaptArgs &a, hipStream_t s, int first_batch, bool offsets_valid,
                       bool prefix_ahead, int max_sweeps, uint32_t epoch, int64_t *host,
-                      int64_t *host_dev, int64_t *seq, AdaptPlan *plan);
+                      int64_t *host_dev, int64_t *seq, const StepArgs *late, AdaptPlan *plan);
 // Refinement flags from surface-elevation jumps to wet neighbours.
 hipError_t flag_eta_jumps(int64_t n, const double *eta, const double *b, const int32_t *nbr,
                           const int8_t *depth, double drytol, double refine_tol,

@@ -283,3 +283,55 @@ def test_long_runs_equal_single_traversals(depth):
             assert np.array_equal(a, b)
     op.close()
     ref.op.close()
+
+
+def test_late_reductions():
+    """On meshes of more than 4096 chunks a single step that nobody waits for
+    leaves its partials to the remeshing after it, or to the next call that
+    needs the slots: steps with and without remeshings between them, single
+    traversals, longer runs and launch shapes against the host's chain."""
+    print("case: depth 19, 128-cell chunks", flush=True)
+    mesh = host.mesh_uniform(19)
+    st = beach(mesh, 5)
+    dt = host.initial_dt(mesh, st, COURANT) * 1e3
+    ops = [swe.EulerTimestep(mesh, scaling=1e3, dry_tolerance=1e-3, courant=COURANT,
+                             min_depth=18, max_depth=20, boundary=swe.BC_WALL)
+           for _ in range(2)]
+    for op in ops:
+        op.set_tuning(128, 0)
+        op.upload(*st)
+    rng = np.random.default_rng(5)
+    op, ref = ops
+    t, fwd = 0.0, False
+
+    def ref_steps(n, t, dt, fwd):
+        for _ in range(n):
+            res = ref.traverse(dt, fwd)
+            t, dt, fwd = t + dt, COURANT * res.dt_cfl, not fwd
+        return t, dt, fwd
+
+    op.run(1, dt, fwd)
+    t, dt, fwd = ref_steps(1, t, dt, fwd)
+    for k in range(8):
+        op.run(1, None, fwd, wait=False)
+        half = 0.5 * dt
+        t, dt, fwd = ref_steps(1, t, dt, fwd)
+        if k == 1:  # the host's dt moves the state, not the device's chain
+            assert op.traverse(half, fwd).dt_cfl == ref.traverse(half, fwd).dt_cfl
+            fwd = not fwd
+        if k in (2, 3, 6):  # a remeshing that changes the mesh, one that does not
+            flags = np.zeros(op.n, np.int8)
+            if k != 3:
+                flags[rng.random(op.n) < 0.01] = 1
+            assert op.adapt(flags)[0] == ref.adapt(flags)[0]
+        if k == 4:
+            op.run(3, None, fwd, wait=False)
+            t, dt, fwd = ref_steps(3, t, dt, fwd)
+        if k == 5:
+            op.set_tuning(256, 0)
+        if k != 0:
+            assert op.run(0, None, fwd) == (t, dt), k
+        for a, b in zip(op.download(), ref.download()):
+            assert np.array_equal(a, b), k
+    for o in ops:
+        o.close()

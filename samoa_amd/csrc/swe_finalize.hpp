@@ -18,9 +18,10 @@ __device__ __forceinline__ double max_f64(double a, double b) {
     return r;
 }
 
-// Lane 63 gets the maximum over the wave of values >= 0 (0 without any; NaN
-// values are left out): row shifts by 1, 2, 4 and 8, then the rows' last lanes
-// broadcast to the next row and half; a lane without a source reads 0.
+// Lane 63 gets the maximum over the wave of values >= 0: row shifts by 1, 2, 4
+// and 8, then the rows' last lanes broadcast to the next row and half; a lane
+// without a source reads 0.  NaN values are left out, but of 64 of them lane 63
+// gets a NaN.
 __device__ __forceinline__ double wave_max(double v) {
     auto step = [&](auto ctrl) {
         constexpr int C = decltype(ctrl)::value;

@@ -508,7 +508,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void eu
         }
         __syncthreads();
         if (t == 0) {
-            double m = s_wmax[0];
+            // from 0: a chunk of NaN sets no limit (meet compares bits, where
+            // a NaN is above every number)
+            double m = max_f64(0.0, s_wmax[0]);
             int rsum = s_wref[0];
 #pragma unroll
             for (int w = 1; w < NW; ++w) {

@@ -343,12 +343,15 @@ __device__ __forceinline__ void edge_flux(double nx, double ny, double hL, doubl
     fR.s = s;
 }
 
-// An edge whose general solve takes no branch that matters, as in
+// An edge whose general solve takes no branch that matters: the test of
 // swe_riemann_clear.hpp (both sides wet: the roots are above 0.06; their bound
-// keeps the test's rounding below its margin, and a NaN or an infinity fails).
+// keeps the test's rounding below its margin), with each velocity compared by
+// itself, so that a NaN or an infinity on either side fails.
 template <int SOLVER>
 __device__ __forceinline__ bool is_clear(double uL, double uR, double sqL, double sqR) {
-    return swe::is_clear<SOLVER>(uL, uR, sqL, sqR) && sqL + sqR < 0x1p26;
+    constexpr double K = SOLVER == 1 ? 0.5 : 2.5;
+    const double m = __builtin_fma(-K, fabs(sqL - sqR), 0.5 * (sqL + sqR));
+    return m - fabs(uL) > 0.06 && m - fabs(uR) > 0.06 && sqL + sqR < 0x1p26;
 }
 
 // edge_flux<SOLVER> on a clear edge: the same operations without riemanntype,

@@ -278,12 +278,18 @@ struct Batch {
     char *stage = nullptr;   // pinned, STAGE_SIZES[stage_size], taken when a transfer needs it
     int stage_size = 0;
     hipEvent_t ring_event[RING_SLOTS] = {};
-    double *d_part_max[2] = {nullptr, nullptr};  // [part_cap] fastest cell per chunk
+    // [part_cap] fastest cell per chunk: two that a chain of steps takes in turn,
+    // and one for every other launch (a caller may replay captured ones while
+    // a chain is pending)
+    double *d_part_max[3] = {nullptr, nullptr, nullptr};
     int32_t *d_part_nref = nullptr;   // [part_cap] refinement count per chunk
     // A chain of steps without finalize kernels (batch_run): the device dt is
     // not in the slots yet, but in the partials of the last step,
     // d_part_max[pp], over the pend_chunks chunks that mesh had.
     bool pending = false;
+    // A caller captured steps of this handle: every run leaves the dt chain in
+    // the slots, where their replays take it from.
+    bool captured = false;
     int pp = 0;
     int64_t pend_chunks = 0;
     int64_t part_cap = 0;
@@ -358,8 +364,7 @@ void release(Batch &B) {
     (void)hipFree(B.d_chunk_scen);
     (void)hipFree(B.d_slots);
     (void)hipFree(B.d_dt);
-    (void)hipFree(B.d_part_max[0]);
-    (void)hipFree(B.d_part_max[1]);
+    for (double *p : B.d_part_max) (void)hipFree(p);
     (void)hipFree(B.d_part_nref);
     (void)hipFree(B.d_meet);
     (void)hipFree(B.d_lists);
@@ -436,16 +441,17 @@ int rebuild_chunks(Batch &B, bool upload = true) {
         const int64_t cap = B.nchunks + B.nchunks / 4;
         SWE_TRY(chain_flush(B));
         if (B.stream) HIP_TRY(hipStreamSynchronize(B.stream));
-        (void)hipFree(B.d_part_max[0]);
-        (void)hipFree(B.d_part_max[1]);
+        for (double *&p : B.d_part_max) {
+            (void)hipFree(p);
+            p = nullptr;
+        }
         (void)hipFree(B.d_part_nref);
-        B.d_part_max[0] = B.d_part_max[1] = nullptr;
         B.d_part_nref = nullptr;
         B.part_cap = 0;
-        if (hipMalloc(&B.d_part_max[0], sizeof(double) * (size_t)cap) != hipSuccess ||
-            hipMalloc(&B.d_part_max[1], sizeof(double) * (size_t)cap) != hipSuccess ||
-            hipMalloc(&B.d_part_nref, sizeof(int32_t) * (size_t)cap) != hipSuccess)
-            return fail(SWE_ERR_NOMEM, "chunk partials allocation failed");
+        bool ok = hipMalloc(&B.d_part_nref, sizeof(int32_t) * (size_t)cap) == hipSuccess;
+        for (double *&p : B.d_part_max)
+            ok = ok && hipMalloc(&p, sizeof(double) * (size_t)cap) == hipSuccess;
+        if (!ok) return fail(SWE_ERR_NOMEM, "chunk partials allocation failed");
         B.part_cap = cap;
     }
     (void)hipFree(B.d_chunk_scen);
@@ -623,7 +629,7 @@ swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
     a.chunk_scen = B.d_chunk_scen;
     a.lists = B.lists_valid ? B.d_lists : nullptr;
     a.slots = B.d_slots;
-    a.part_max = B.d_part_max[1 - B.pp];  // not the one a chain may still need
+    a.part_max = B.d_part_max[2];
     a.part_nref = B.d_part_nref;
     a.n_scen = B.nscen;
     a.nchunks = B.nchunks;
@@ -931,19 +937,21 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (!own) HIP_TRY(hipStreamIsCapturing(B.stream, &capture));
     const bool captured = capture != hipStreamCaptureStatusNone;
+    B.captured = B.captured || captured;
     if (!captured) SWE_TRY(lists_for(B, n_steps));
     // Meshes of few chunks step in a chain: a step forms its dt from the
     // partials of the one before, and a finalize kernel runs only for who
-    // reads the results.  On a caller's stream the chain ends with the call (so
-    // that a capture finds the slots current), which a short one isn't worth.
-    bool chain = own || (!captured && n_steps >= CHAIN_LEAST);
+    // reads the results.  On a caller's stream, and after a capture, the chain
+    // ends with the call (so that captured steps find the slots current), which
+    // a short one isn't worth.
+    bool chain = (own && !B.captured) || (!captured && n_steps >= CHAIN_LEAST);
     for (auto &s : B.scen) chain = chain && s.nchunks <= swe::CHAIN_CHUNKS;
     if (!chain) SWE_TRY(chain_flush(B));
     // A single step of a larger mesh that nobody waits for leaves its partials too:
     // a remeshing that follows finalizes them beside a kernel of its own, any
     // other call before it reads the slots.
-    const bool late = own && !chain && B.nscen == 1 && n_steps == 1 && !time && !dt_next &&
-                      !meet_of(B);
+    const bool late = own && !B.captured && !chain && B.nscen == 1 && n_steps == 1 && !time &&
+                      !dt_next && !meet_of(B);
     // one step from state buffer `from`; in a chain, with the partials
     // d_part_max[pp] of the step before if there is one
     auto one_step = [&](hipStream_t st, int from, int fwd, bool prev, int pp) -> hipError_t {
@@ -1020,7 +1028,7 @@ int batch_run(Batch &B, int64_t n_steps, const double *dt0, int forward, double 
     }
     while (left > 0) SWE_TRY(single());
     if (n_steps > 0) B.flags_valid = B.keep_flags != 0;
-    if (!own || time || dt_next) SWE_TRY(chain_flush(B));
+    if (!own || B.captured || time || dt_next) SWE_TRY(chain_flush(B));
     if (!time && !dt_next) return SWE_OK;
     std::vector<swe::Slots> res((size_t)B.nscen);
     const Part part{B.d_slots, res.data(), sizeof(swe::Slots) * res.size()};

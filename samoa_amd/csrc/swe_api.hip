@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "swe_internal.hpp"
+#include "swe_list_rule.hpp"
 #include "swe_sweep_stamp.hpp"
 #include "swe_mi355x.h"
 #include "swe_riemann.hpp"
@@ -237,9 +238,6 @@ void stage_give(int k, char *p) {
     (void)hipHostFree(p);
 }
 
-// Traversals of a changed mesh after which its edge lists are stored.
-constexpr int64_t LISTS_FROM = 2;
-
 // Steps of a captured graph (an even number: the state's buffers, the direction
 // and the partials are then where they were), and of a run that is worth it.  A
 // graph launch costs the device 3-4 us, a launch from the host 0.4 us more than
@@ -249,6 +247,7 @@ constexpr int64_t LISTS_FROM = 2;
 // capture 1160 us in twos, 905 one by one, 970 in graphs of 24).
 constexpr int GRAPH_STEPS = 24;
 constexpr int64_t GRAPH_FROM = 2 * GRAPH_STEPS;
+static_assert(GRAPH_FROM >= swe::lists_break_even(0), "graphs are captured with the lists");
 
 // Steps of a run on a caller's stream from which they form a chain: it saves
 // about 1 us a step against workgroups that meet, its end costs 4 us.
@@ -265,10 +264,14 @@ struct Batch {
     std::vector<swe::Scen> scen;
     std::vector<int> uniform_depth;
     int64_t ncells = 0, ntopo = 0, nchunks = 0;
-    uint32_t *d_lists = nullptr;  // the chunks' edge lists (lists_valid), of lists_cap bytes
-    size_t lists_cap = 0;
-    bool lists_valid = false;
-    int64_t list_uses = 0;  // traversals since the mesh or the chunks changed
+    // The chunks' edge lists (lists_valid), with room for a mesh of `cap` cells
+    // at every chunk size; null: there was no memory, steps build their own.
+    // Queued on `stream`: lists_event follows, lists_done once it was seen.
+    uint32_t *d_lists = nullptr;
+    hipEvent_t lists_event = nullptr;
+    bool lists_valid = false, lists_done = false;
+    // steps of swe_step and swe_run on this mesh, and on the one before it
+    int64_t list_uses = 0, list_uses_before = 0;
     int chunk = swe::DEFAULT_CHUNK;
     int64_t grid = 0;
     swe::Scen *d_scen = nullptr;
@@ -368,6 +371,7 @@ void release(Batch &B) {
     (void)hipFree(B.d_part_nref);
     (void)hipFree(B.d_meet);
     (void)hipFree(B.d_lists);
+    if (B.lists_event) (void)hipEventDestroy(B.lists_event);
     (void)hipFree(B.b2);
     (void)hipFree(B.nbr2);
     (void)hipFree(B.plotter2);
@@ -471,41 +475,69 @@ int rebuild_chunks(Batch &B, bool upload = true) {
                                hipMemcpyHostToDevice, B.stream));
     drop_graphs(B);
     B.lists_valid = false;
-    B.list_uses = 0;
     return SWE_OK;
 }
 
-// Stores the chunks' edge lists, on the handle's stream, and waits for them:
-// from then on any stream's steps may read them.  A mesh keeps its lists until
-// it or the chunk size changes.  Without the memory for them, steps build
-// their own.
-int store_lists(Batch &B) {
-    if (B.lists_valid) return SWE_OK;
-    const size_t bytes = swe::edge_list_bytes(B.nchunks, B.chunk);
-    if (bytes > B.lists_cap) {
-        (void)hipFree(B.d_lists);
-        B.d_lists = nullptr;
-        B.lists_cap = 0;
-        if (hipMalloc(&B.d_lists, bytes + bytes / 8) != hipSuccess) {
-            B.d_lists = nullptr;
-            (void)hipGetLastError();
-            return SWE_OK;
-        }
-        B.lists_cap = bytes + bytes / 8;
+// Room for the edge lists of a single mesh of up to `cells` cells, or of the
+// batch's meshes, at every chunk size: replays of captured steps may read them
+// for as long as the handle keeps its buffers.  Called while nothing runs.
+void alloc_lists(Batch &B, int64_t cells) {
+    (void)hipFree(B.d_lists);
+    B.d_lists = nullptr;
+    B.lists_valid = false;
+    size_t bytes = 0;
+    for (int chunk : swe::CHUNK_SIZES) {
+        int64_t chunks = 0;
+        if (B.nscen == 1) chunks = (cells + chunk - 1) / chunk;
+        else for (auto &s : B.scen) chunks += (s.n + chunk - 1) / chunk;
+        bytes = std::max(bytes, swe::edge_list_bytes(chunks, chunk));
     }
-    drop_graphs(B);  // captured without lists
+    if (hipMalloc(&B.d_lists, bytes) != hipSuccess) {
+        B.d_lists = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
+// Stores the chunks' edge lists, on the handle's stream.  A mesh keeps its
+// lists until it or the chunk size changes.
+int store_lists(Batch &B) {
+    if (B.lists_valid || !B.d_lists) return SWE_OK;
+    if (!B.lists_event) HIP_TRY(hipEventCreateWithFlags(&B.lists_event, hipEventDisableTiming));
     HIP_TRY(swe::build_edge_lists(make_args(B, 0, 1, 1), B.chunk, B.d_lists, B.stream));
-    HIP_TRY(hipStreamSynchronize(B.stream));
+    HIP_TRY(hipEventRecord(B.lists_event, B.stream));
     B.lists_valid = true;
+    B.lists_done = false;
     return SWE_OK;
 }
 
-// Before `steps` traversals of the handle's state: a changed mesh is worth its
-// lists once several traversals use them (building takes about what two save).
-int lists_for(Batch &B, int64_t steps) {
-    B.list_uses += steps;
-    if (!B.lists_valid && B.list_uses > LISTS_FROM) SWE_TRY(store_lists(B));
+int store_lists_now(Batch &B) {
+    SWE_TRY(store_lists(B));
+    HIP_TRY(hipStreamSynchronize(B.stream));
+    B.lists_done = true;
     return SWE_OK;
+}
+
+// The lists for a launch on stream `st`: on another one than the handle's only
+// once they are known to be there (a wait for them would not fit a capture).
+const uint32_t *lists_on(Batch &B, hipStream_t st) {
+    if (!B.lists_valid) return nullptr;
+    if (st != B.stream && !B.lists_done) {
+        if (hipEventQuery(B.lists_event) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        B.lists_done = true;
+    }
+    return B.d_lists;
+}
+
+// Before `steps` steps of swe_step or swe_run: stores the lists of a changed mesh
+// when that pays.  (Traversals on device pointers use lists that are there, but
+// do not store any: theirs may be any stream, and captured.)
+int lists_for(Batch &B, int64_t steps) {
+    const bool store = swe::lists_pay(B.ncells, B.list_uses, steps, B.list_uses_before);
+    B.list_uses += steps;
+    return store ? store_lists(B) : SWE_OK;
 }
 
 int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
@@ -609,7 +641,8 @@ int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
     B.uploaded.assign((size_t)nscen, 0);
     B.cap = B.ncells;
     SWE_TRY(rebuild_chunks(B));
-    return store_lists(B);
+    alloc_lists(B, B.ncells);
+    return store_lists_now(B);
 }
 
 swe::StepArgs make_args(const Batch &B, int from, int to, int forward) {
@@ -1307,6 +1340,7 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
         B.refine = ro;
         B.cur = 0;
         B.cap = cap;
+        alloc_lists(B, cap);
     } else {
         std::swap(B.b, B.b2);
         std::swap(B.nbr, B.nbr2);
@@ -1321,6 +1355,8 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
     B.scen[0] = sn;
     B.uniform_depth[0] = -1;
     B.flags_valid = false;
+    B.list_uses_before = B.list_uses;
+    B.list_uses = 0;
     SWE_TRY(rebuild_chunks(B, false));
     if (n_out) *n_out = n_new;
     if (sweeps_out) *sweeps_out = sweeps;
@@ -1358,6 +1394,7 @@ int batch_forward_device(Batch &B, const double *eta, const double *hu, const do
     a.out_dtcfl = dt_cfl_dev;
     a.skip_finalize = dt_cfl_dev ? 0 : 1;  // dt comes from the caller: no result is read
     a.meet = dt_cfl_dev ? meet_of(B) : nullptr;
+    a.lists = lists_on(B, st);
     a.tol = 0;  // the adjoint's sweeps: the rounding its kernels differentiate
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, st));
     return SWE_OK;
@@ -1393,7 +1430,7 @@ int batch_adjoint_device(Batch &B, const double *eta, const double *hu, const do
     a.scen = B.d_scen;
     a.chunk_scen = B.d_chunk_scen;
     a.nchunks = B.nchunks;
-    a.lists = B.lists_valid ? B.d_lists : nullptr;
+    a.lists = lists_on(B, st);
     a.dt_dev = dt_dev;
     a.g = B.g;
     a.inv16g = 1.0 / (16.0 * B.g);
@@ -1433,7 +1470,7 @@ int batch_set_tuning(Batch &B, int chunk, int64_t grid) {
     if (chunk != B.chunk) {
         B.chunk = chunk;
         SWE_TRY(rebuild_chunks(B));
-        SWE_TRY(store_lists(B));
+        SWE_TRY(store_lists_now(B));
     }
     return SWE_OK;
 }
@@ -1666,6 +1703,7 @@ int swe_step_device(swe_handle *h, const double *eta, const double *hu, const do
     a.out_dtcfl = dt_cfl_dev;
     a.out_nref = n_refine_dev;
     a.meet = meet_of(B);
+    a.lists = lists_on(B, s);
     HIP_TRY(swe::launch_step(a, B.solver, B.chunk, B.grid, s));
     return SWE_OK;
 }

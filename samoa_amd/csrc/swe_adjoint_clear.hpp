@@ -21,8 +21,9 @@ namespace swe {
 // Seeds gfL/gfR on (h, hu, hv) of the left and right fluxes; gradients with
 // respect to (eta, hu, hv, b) of both sides.  rL, cL: 1/h and sqrt(g h) of
 // clear_cell; e: clear_edge.  Returns false, with nothing valid in the
-// gradients, if a bound on the steady-state jump may be taken.
-template <int SOLVER>
+// gradients, if a bound on the steady-state jump may be taken (WAVE: in any of
+// the wave's lanes that are here).
+template <int SOLVER, bool WAVE = false>
 SWE_HD bool clear_flux_adj(double nx, double ny, const ClearEdge &e, double hL, double bL,
                            double rL, double cL, double hR, double bR, double rR, double cR,
                            double g, const double gfL[3], const double gfR[3], double gQL[4],
@@ -89,7 +90,11 @@ SWE_HD bool clear_flux_adj(double nx, double ny, const ClearEdge &e, double hL, 
         const double M = (delb * g) * hbar;
         const double deldelh = div_near(M, s1s2bar, ib);
         const double n = ((e.pL - e.pR) + l2 * hR) - l0 * hL;
-        if (!(fmax(deldelh * l0, deldelh * l2) < n * (1.0 - 0x1p-40))) return false;
+        bool bounded = !(fmax(deldelh * l0, deldelh * l2) < n * (1.0 - 0x1p-40));
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (WAVE) bounded = __ballot(bounded) != 0;
+#endif
+        if (bounded) return false;
         const double Kp = M * s1s2tilde;
         const double p0 = -div_near(Kp, s1s2bar, ib);
         const double pL = -(hL * delb), pR = -(hR * delb);

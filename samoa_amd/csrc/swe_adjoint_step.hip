@@ -12,9 +12,9 @@
 // Transpose update: the limiter passes the adjoint through, or stops it
 // where a fix overwrote a value; the flux sum dQ = s * sum_k len_k f_k
 // (s = -dt / vol) then seeds every edge flux of the cell with s * len_k * lam.
-// Transpose flux: each edge of the chunk's compacted edge list (the same
-// list the forward kernel builds) runs edge_flux_adj with the seeds of both
-// cells, and the gradients with respect to both states are written to
+// Transpose flux: each edge of the chunk's compacted edge list (the forward
+// kernel's, stored with the mesh or built here) runs edge_flux_adj with the seeds
+// of both cells, and the gradients with respect to both states are written to
 // per-(cell, edge) LDS slots, summed per cell in a fixed order (so results do
 // not depend on scheduling).  Edges to cells of other chunks are solved by
 // both chunks, each keeping its own side.
@@ -28,7 +28,13 @@
 // registers: held to 168 it spills 76 bytes on its few edges, and three waves
 // per SIMD instead of two hide more of the first pass's LDS and memory waits:
 // 213.7 us with neither, 122 with two waves, 106 with three.  LDS (50 KB for
-// 256 cells) allows no fourth.  The f-wave kernel went from 107 to 81 us.
+// 256 cells) allows no fourth.  The f-wave kernel went from 107 to 81 us.  A mesh
+// of nothing but general edges pays for the first pass: 79 -> 92 us at 524 k cells
+// (f-wave 36 -> 42).
+//
+// Meshes that do not fill the chip are as long as their slowest chunk, and take
+// one pass (launch_adj_t): a wave with a general edge solves all of its edges
+// so, and there is neither a second list nor a barrier between the passes.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -46,9 +52,10 @@ __constant__ double c_normal_adj[17 * 3 * 2];  // [plotter + 8][edge][x,y]
 __constant__ double c_leg_adj[64];             // l(k) = sqrt(0.5)**k at k + 1
 
 // NT threads work on a chunk, CH or 2 CH; the first CH hold a cell each.  512 of
-// them fill two waves per SIMD, as does the LDS of 512 cells.
-template <int SOLVER, int CH, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 ? 2 : 3))) void
+// them fill two waves per SIMD, as does the LDS of 512 cells.  ONE: a single
+// pass over the list, with the general solver's registers.
+template <int SOLVER, int CH, int NT, bool ONE>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(ONE || NT == 512 ? 2 : 3))) void
 adjoint_step_kernel(AdjArgs args) {
     __shared__ double s_q[4][CH];     // eta, hu, hv, b of the chunk at t_n
     __shared__ double s_x[2][CH];     // 1/h and sqrt(g h) of each cell (clear_cell)
@@ -56,7 +63,7 @@ adjoint_step_kernel(AdjArgs args) {
     __shared__ double s_gb[CH];       // each cell's b gradient so far
     __shared__ double s_g[4][3][CH];  // transpose-flux contributions per (edge, cell)
     __shared__ uint32_t s_list[3 * CH + 4];  // the edge list (swe_device.hpp)
-    __shared__ uint16_t s_rest[3 * CH];  // entries left to the general solver
+    __shared__ uint16_t s_rest[ONE ? 1 : 3 * CH];  // entries left to the general solver
     __shared__ int8_t s_dep[CH], s_mask[CH];
     __shared__ int s_wsum[NT / 64], s_nrest;
     __shared__ double s_dir[8][2];  // the unit vectors at multiples of 45 degrees
@@ -152,7 +159,8 @@ adjoint_step_kernel(AdjArgs args) {
 
         __builtin_amdgcn_s_setprio(0);
         // One pass over the list (FIRST, clear_flux_adj; it lists the edges
-        // that are not clear) or over the rest (edge_flux_adj).  An edge's
+        // that are not clear, or solves them if it is the only one) or over
+        // the rest (edge_flux_adj).  An edge's
         // pass depends on its two states alone and each writes its own
         // slots, so results depend neither on the chunking nor on the order
         // of the rest.  Two passes: the general solver's registers do not
@@ -253,7 +261,19 @@ adjoint_step_kernel(AdjArgs args) {
             if constexpr (FIRST) {
                 const double hL = L[0] - L[3], hR = R[0] - R[3];
                 const ClearEdge ce = clear_edge(nx, ny, hL, L[1], L[2], L[4], hR, R[1], R[2], R[4]);
-                if (is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5])) {
+                if constexpr (ONE) {
+                    // a wave with a general edge solves all of its edges so
+                    const bool clear = is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5]);
+                    bool general =
+                        __ballot(!clear && !(hL <= drytol && hR <= drytol)) != 0;
+                    if (clear && !general)
+                        general = !clear_flux_adj<SOLVER, true>(nx, ny, ce, hL, L[3], L[4], L[5],
+                                                                hR, R[3], R[4], R[5], g, fL, fR,
+                                                                gL, gR);
+                    if (general)
+                        edge_flux_adj<SOLVER>(nx, ny, L[0], L[1], L[2], L[3], R[0], R[1], R[2],
+                                              R[3], drytol, g, a.inv16g, fL, fR, gL, gR);
+                } else if (is_clear<SOLVER>(ce.uL, ce.uR, L[5], R[5])) {
                     if (!clear_flux_adj<SOLVER>(nx, ny, ce, hL, L[3], L[4], L[5], hR, R[3], R[4],
                                                 R[5], g, fL, fR, gL, gR)) {
                         s_rest[atomicAdd(&s_nrest, 1)] = (uint16_t)e;
@@ -293,10 +313,12 @@ adjoint_step_kernel(AdjArgs args) {
         };
         solve(std::true_type{}, total);
         __syncthreads();
-        const int nrest = s_nrest;
-        if (nrest) {
-            solve(std::false_type{}, nrest);
-            __syncthreads();
+        if constexpr (!ONE) {
+            const int nrest = s_nrest;
+            if (nrest) {
+                solve(std::false_type{}, nrest);
+                __syncthreads();
+            }
         }
 
         asm volatile("" : "+v"(t));
@@ -342,17 +364,43 @@ static void launch_adj_t(const AdjArgs &a, int64_t grid_blocks, hipStream_t s) {
     const int64_t blocks = grid_blocks > 0 && grid_blocks < nvirt ? grid_blocks : nvirt;
     // Two threads per cell where every workgroup is resident at once that way (256
     // CUs of 512 lanes): a chunk's ~1.6 CH edges then take one round, and the
-    // general solver keeps its 205 registers.  A launch, us: 13.8 -> 11.9 at 8
-    // chunks, 15.0 -> 12.8 at 256, with 128-cell chunks 16.9 -> 14.6 at 512, the
-    // f-wave solver 9.0 -> 8.3 at 256; but 17.4 -> 20.9 at 512 chunks, 24.2 -> 31.7
-    // at 1024.
+    // general solver keeps its 205 registers.  A launch of the augmented solver,
+    // us: 13.8 -> 11.9 at 8 chunks, 15.0 -> 12.8 at 256, with 128-cell chunks
+    // 16.9 -> 14.6 at 512; but 17.4 -> 20.9 at 512 chunks, 24.2 -> 31.7 at 1024.
+    //
+    // One pass where all are resident (two waves per SIMD) and the launch is as
+    // long as a chunk that would pay both: us a launch on a beach (a third of its
+    // edges general) with two passes / with one,
+    //     f-wave, 256-cell chunks: 1: 6.1 / 4.8, 32: 8.0 / 6.9, 128: 8.2 / 7.0,
+    //       256: 8.1 / 7.1, 512: 10.5 / 9.9; every edge general 9.8 / 6.9 at 32,
+    //       15.3 / 12.0 at 512; none 5.3 / 5.2 and 8.2 / 8.1
+    //     augmented: 1: 10.0 / 8.5, 512: 18.1 / 17.2 (every edge 30.8 / 23.8); with
+    //       128-cell chunks 128: 12.7 / 10.8, 512: 16.6 / 12.6
+    // With two threads per cell of 256-cell chunks the augmented solver's long
+    // branches tell, which a wave in one pass takes for its clear edges too: 12.1 /
+    // 13.9 at 4 chunks, 12.3 / 13.9 at 128, 12.9 / 12.8 at 256, and 512-cell chunks
+    // 15.6 / 14.1 to 15.7 / 22.3: two passes there.
     constexpr int TWO = CH <= 256 ? 2 * CH : CH;
-    if (CH <= 256 && a.nchunks * TWO <= 256 * 512)
-        hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH, TWO>), dim3((unsigned)blocks),
-                           dim3(TWO), 0, s, a);
-    else
-        hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH, CH>), dim3((unsigned)blocks), dim3(CH),
-                           0, s, a);
+    constexpr bool SHORT = SOLVER == 1 || CH == 128;
+    const int64_t resident = 256 * 512;
+    const dim3 grid((unsigned)blocks);
+    auto launch = [&](auto threads, auto one) {
+        constexpr int NT = decltype(threads)::value;
+        constexpr bool ONE = decltype(one)::value;
+        hipLaunchKernelGGL((adjoint_step_kernel<SOLVER, CH, NT, ONE>), grid, dim3(NT), 0, s, a);
+    };
+    using two_threads = std::integral_constant<int, TWO>;
+    using one_thread = std::integral_constant<int, CH>;
+    if constexpr (CH <= 256) {
+        if (a.nchunks * TWO <= resident) {
+            if (SHORT || a.nchunks == 1) return launch(two_threads{}, std::true_type{});
+            if constexpr (!SHORT) return launch(two_threads{}, std::false_type{});
+        }
+    }
+    if constexpr (SHORT || CH == 256) {
+        if (a.nchunks * CH <= resident) return launch(one_thread{}, std::true_type{});
+    }
+    launch(one_thread{}, std::false_type{});
 }
 
 hipError_t launch_adjoint(const AdjArgs &a, int solver, int chunk, int64_t grid_blocks,

@@ -120,9 +120,12 @@ int swe_run(swe_handle *h, int64_t n_steps, double dt0, int forward, double dt_c
 
 /* The device's null stream (whose hipStream_t is NULL) as a `stream` argument
  * of swe_step_device, swe_forward_device, swe_adjoint_step_device,
- * swe_adapt_record_device and their batch forms.  A caller whose own work is on
- * the null stream names it so: the library's stream is ordered with it too,
- * but each change from one to the other costs 25-30 us. */
+ * swe_adapt_record_device and their batch forms, where NULL is the library's
+ * stream.  A caller whose own work is on the null stream names it so: the
+ * library's stream is ordered with it too, but each change from one to the
+ * other costs 25-30 us.  swe_step_device_noalloc and swe_transfer_adjoint_device
+ * take it as they take NULL; swe_set_stream and swe_batch_set_stream refuse it
+ * (SWE_ERR_ARG). */
 #define SWE_STREAM_NULL ((void *)1)
 
 /* Device-pointer step for callers that own device memory (the PyTorch

@@ -1364,10 +1364,12 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
 }
 
 // The stream that a caller names: NULL the handle's, SWE_STREAM_NULL the
-// device's null stream.
+// device's null stream, which is also what a call without a handle takes for NULL.
+hipStream_t stream_of(void *stream) {
+    return stream == SWE_STREAM_NULL ? nullptr : (hipStream_t)stream;
+}
 hipStream_t stream_of(const Batch &B, void *stream) {
-    if (stream == SWE_STREAM_NULL) return nullptr;
-    return stream ? (hipStream_t)stream : B.stream;
+    return stream ? stream_of(stream) : B.stream;
 }
 
 // Forward traversal on caller-owned device buffers (all scenarios), dt read
@@ -1444,6 +1446,9 @@ int batch_adjoint_device(Batch &B, const double *eta, const double *hu, const do
 }
 
 int batch_set_stream(Batch &B, void *stream) {
+    if (stream == SWE_STREAM_NULL)
+        return fail(SWE_ERR_ARG, "set_stream: a handle cannot launch on the null stream (NULL "
+                    "names its own, which is ordered with it)");
     SWE_TRY(chain_flush(B));
     HIP_TRY(hipStreamSynchronize(B.stream));
     B.stream = stream ? (hipStream_t)stream : B.own_stream;
@@ -1642,7 +1647,7 @@ int swe_transfer_adjoint_device(int64_t n_old, const int8_t *code, const int64_t
         !lhv_out || !gb_out)
         return fail(SWE_ERR_ARG, "swe_transfer_adjoint_device: invalid argument");
     HIP_TRY(swe::transfer_adjoint(n_old, code, base, b_sampled, leta, lhu, lhv, gb, leta_out,
-                                  lhu_out, lhv_out, gb_out, (hipStream_t)stream));
+                                  lhu_out, lhv_out, gb_out, stream_of(stream)));
     return SWE_OK;
 }
 
@@ -1842,7 +1847,7 @@ int swe_step_device_noalloc(const swe_device_mesh *m, const double *eta, const d
     sc.depth = -1;
     sc.dmin = m->min_depth;
     sc.dmax = m->max_depth;
-    HIP_TRY(swe::launch_step_raw(a, m->solver, (hipStream_t)stream));
+    HIP_TRY(swe::launch_step_raw(a, m->solver, stream_of(stream)));
     return SWE_OK;
 }
 

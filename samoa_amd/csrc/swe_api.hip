@@ -264,12 +264,12 @@ struct Batch {
     std::vector<swe::Scen> scen;
     std::vector<int> uniform_depth;
     int64_t ncells = 0, ntopo = 0, nchunks = 0;
-    // The chunks' edge lists (lists_valid), with room for a mesh of `cap` cells
-    // at every chunk size; null: there was no memory, steps build their own.
-    // Queued on `stream`: lists_event follows, lists_done once it was seen.
+    // The chunks' edge lists (lists_valid), queued on `stream`: lists_event
+    // follows, lists_done once it was seen.  lists_refused: there was no memory,
+    // and steps build their own until the buffers grow.
     uint32_t *d_lists = nullptr;
     hipEvent_t lists_event = nullptr;
-    bool lists_valid = false, lists_done = false;
+    bool lists_valid = false, lists_done = false, lists_refused = false;
     // steps of swe_step and swe_run on this mesh, and on the one before it
     int64_t list_uses = 0, list_uses_before = 0;
     int chunk = swe::DEFAULT_CHUNK;
@@ -478,22 +478,20 @@ int rebuild_chunks(Batch &B, bool upload = true) {
     return SWE_OK;
 }
 
-// Room for the edge lists of a single mesh of up to `cells` cells, or of the
-// batch's meshes, at every chunk size: replays of captured steps may read them
-// for as long as the handle keeps its buffers.  Called while nothing runs.
-void alloc_lists(Batch &B, int64_t cells) {
-    (void)hipFree(B.d_lists);
-    B.d_lists = nullptr;
-    B.lists_valid = false;
+// Room for the edge lists of the handle's mesh, as large as it can get in its
+// buffers, or of the batch's meshes, at every chunk size: replays of captured steps
+// may read them for as long as the handle keeps those buffers.
+void alloc_lists(Batch &B) {
     size_t bytes = 0;
     for (int chunk : swe::CHUNK_SIZES) {
         int64_t chunks = 0;
-        if (B.nscen == 1) chunks = (cells + chunk - 1) / chunk;
+        if (B.nscen == 1) chunks = (B.cap + chunk - 1) / chunk;
         else for (auto &s : B.scen) chunks += (s.n + chunk - 1) / chunk;
         bytes = std::max(bytes, swe::edge_list_bytes(chunks, chunk));
     }
     if (hipMalloc(&B.d_lists, bytes) != hipSuccess) {
         B.d_lists = nullptr;
+        B.lists_refused = true;
         (void)hipGetLastError();
     }
 }
@@ -501,7 +499,9 @@ void alloc_lists(Batch &B, int64_t cells) {
 // Stores the chunks' edge lists, on the handle's stream.  A mesh keeps its
 // lists until it or the chunk size changes.
 int store_lists(Batch &B) {
-    if (B.lists_valid || !B.d_lists) return SWE_OK;
+    if (B.lists_valid) return SWE_OK;
+    if (!B.d_lists && !B.lists_refused) alloc_lists(B);
+    if (!B.d_lists) return SWE_OK;
     if (!B.lists_event) HIP_TRY(hipEventCreateWithFlags(&B.lists_event, hipEventDisableTiming));
     HIP_TRY(swe::build_edge_lists(make_args(B, 0, 1, 1), B.chunk, B.d_lists, B.stream));
     HIP_TRY(hipEventRecord(B.lists_event, B.stream));
@@ -641,7 +641,6 @@ int batch_init(Batch &B, int32_t nscen, const swe_mesh_desc *descs) {
     B.uploaded.assign((size_t)nscen, 0);
     B.cap = B.ncells;
     SWE_TRY(rebuild_chunks(B));
-    alloc_lists(B, B.ncells);
     return store_lists_now(B);
 }
 
@@ -1340,7 +1339,9 @@ int batch_adapt(Batch &B, const int8_t *refine_host, int64_t *n_out, int *sweeps
         B.refine = ro;
         B.cur = 0;
         B.cap = cap;
-        alloc_lists(B, cap);
+        (void)hipFree(B.d_lists);  // of the old buffers' size
+        B.d_lists = nullptr;
+        B.lists_refused = B.lists_valid = false;
     } else {
         std::swap(B.b, B.b2);
         std::swap(B.nbr, B.nbr2);

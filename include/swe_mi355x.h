@@ -110,8 +110,9 @@ int swe_step(swe_handle *h, double dt, int forward, double *dt_cfl, int64_t *n_r
  * disables the clamp).  The direction starts at `forward` and flips after
  * every step.  *time is the simulated time before the steps on entry and is
  * advanced by each step's dt on the device (t = t + dt, in the reference's
- * order); *dt_next receives the dt of the next step.  The steps are captured
- * once into a HIP graph and replayed.
+ * order); *dt_next receives the dt of the next step.  Runs of 48 steps
+ * on replay a HIP graph of 24, captured once; the others, and the rest, are
+ * launched one by one.
  * dt0 <= 0 continues the device chain (dt and time) where the last swe_run
  * left it; *time is then not read.  With time and dt_next both NULL the call
  * returns without waiting for the steps (time is required when dt0 > 0). */
@@ -310,7 +311,9 @@ int swe_set_stream(swe_handle *h, void *stream);
 
 /* Launch shape of the handle's step kernel, as swe_batch_set_tuning below:
  * chunk_cells in {128, 256, 512}, grid_blocks 0 or a multiple of 8.  No
- * counterpart in the reference; results do not depend on it. */
+ * counterpart in the reference; results do not depend on it.  Calls that the
+ * caller captured hold the chunk tables and the mesh: another chunk size, like
+ * a swe_adapt, means capturing them again. */
 int swe_set_tuning(swe_handle *h, int chunk_cells, int64_t grid_blocks);
 int swe_get_tuning(swe_handle *h, int *chunk_cells, int64_t *grid_blocks);
 
@@ -364,8 +367,8 @@ int swe_batch_download(swe_batch *b, int32_t scenario, double *eta, double *hu, 
 int swe_batch_step(swe_batch *b, const double *dt, int forward, double *dt_cfl,
                    int64_t *n_refine);
 /* n_steps traversals of every scenario with per-scenario device dt chains, as
- * swe_run per scenario: dt0[s] and time[s] (in/out), dt_next[s] out.  The
- * steps are replayed from a captured HIP graph. */
+ * swe_run per scenario: dt0[s] and time[s] (in/out), dt_next[s] out, launched
+ * and replayed as there. */
 int swe_batch_run(swe_batch *b, int64_t n_steps, const double *dt0, int forward,
                   double dt_clamp, double *time, double *dt_next);
 /* Launch shape: chunk_cells in {128, 256, 512} (cells per workgroup, one LDS

@@ -4,8 +4,8 @@
 // double-buffered and concatenated, topology shared between scenarios that
 // pass the same mesh arrays), the per-scenario table the step kernel reads,
 // and the reference's dt bookkeeping either on the host (swe_step,
-// swe_batch_step) or on the device inside a captured HIP graph (swe_run,
-// swe_batch_run).  A single-mesh handle is a batch of one.
+// swe_batch_step) or on the device (swe_run, swe_batch_run; long runs replay a
+// captured HIP graph).  A single-mesh handle is a batch of one.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

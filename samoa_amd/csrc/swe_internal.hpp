@@ -223,7 +223,8 @@ hipError_t upload_tables_adjoint(const double *normal, const double *leg);
 hipError_t launch_adjoint(const AdjArgs &a, int solver, int chunk, int64_t grid_blocks,
                           hipStream_t s);
 // Launches the step kernel and, after it on the same stream, the finalize
-// kernel (per-scenario reduction of the chunk partials, results, dt chain).
+// kernel (per-scenario reduction of the chunk partials, results, dt chain), unless
+// its workgroups meet (meet) or the partials are left as they are (skip_finalize).
 // grid_blocks: number of workgroups (multiple of 8) or 0 for one per chunk.
 hipError_t launch_step(const StepArgs &a, int solver, int chunk, int64_t grid_blocks,
                        hipStream_t s);
